@@ -84,7 +84,7 @@ enum {
 enum { LMOE_SCORING_SOFTMAX = 0, LMOE_SCORING_SIGMOID = 1 };
 
 /* Kernel-path selectors of lmoe_grouped_mlp. */
-enum { LMOE_PATH_AUTO = 0, LMOE_PATH_GEMV = 1, LMOE_PATH_MFMA = 2 };
+enum { LMOE_PATH_AUTO = 0, LMOE_PATH_GEMV = 1, LMOE_PATH_MFMA = 2, LMOE_PATH_STREAM = 3 };
 
 /* Slots of the meta[] output of lmoe_permute. */
 enum {
@@ -302,9 +302,12 @@ int lmoe_gather_rows(const void* x, int H, int k, const int32_t* sorted_pairs,
  * indexed by flat pair (rows of unplaced pairs are left untouched).
  * path = LMOE_PATH_GEMV (weight-streaming, small slot groups),
  * LMOE_PATH_MFMA (bf16 MFMA tiles, block_m must equal the block_m given to
- * lmoe_permute: 320 = one workgroup per CU with equal shares of 32-column
+ * lmoe_permute: 64 = weight streaming for few pairs per slot, a row tile per
+ * workgroup, 320 = one workgroup per CU with equal shares of 32-column
  * blocks of 320-row tiles, 256 = a grid of 256 x 256 tiles, 128 = 128 x 128
- * tiles; 320 needs H % 64 == 0) or
+ * tiles; 320 and 64 need H % 64 == 0),
+ * LMOE_PATH_STREAM (the block_m 64 kernel with partial sums of 256 columns:
+ * other bits than LMOE_PATH_MFMA, accumulation as accurate as the GEMVs') or
  * LMOE_PATH_AUTO.  H % 8 == 0, I % 64 == 0.  Every block_m gives the same
  * bits. */
 int lmoe_grouped_mlp(const void* x, int T, int H, int I, int k,
@@ -353,6 +356,23 @@ int lmoe_decode_mlp_two_passes(const void* x, int T, int H, int I, int k,
                                const void* w13_b, const void* w2_b, int n_slots_b,
                                const int32_t* offsets_b, const int32_t* sorted_pairs_b,
                                const int32_t* active_b, int n_pairs, void* act, void* y,
+                               hipStream_t stream);
+
+/* lmoe_decode_mlp_two_passes on the weight-streaming MFMA kernel, for layers
+ * past the GEMVs' token count: the same passes, act rows and disjoint tables,
+ * tile_off in place of active, both permutations built with block_m 64.
+ * path is LMOE_PATH_MFMA or LMOE_PATH_STREAM: every value has the bits of
+ * lmoe_grouped_mlp with that path over each pass.
+ * H % 64 == 0, I % 64 == 0, n_pairs * max(H, I) below 2^31, every operand
+ * 16-byte aligned; else LMOE_ERR_SHAPE. */
+int lmoe_stream_mlp_two_passes(const void* x, int T, int H, int I, int k,
+                               const void* w13_a, const void* w2_a, int n_slots_a,
+                               const int32_t* offsets_a, const int32_t* sorted_pairs_a,
+                               const int32_t* tile_off_a, const int32_t* meta_a,
+                               const void* w13_b, const void* w2_b, int n_slots_b,
+                               const int32_t* offsets_b, const int32_t* sorted_pairs_b,
+                               const int32_t* tile_off_b, const int32_t* meta_b,
+                               int n_pairs, int path, void* act, void* y,
                                hipStream_t stream);
 
 /* Weighted combine: out[t] = sum_{j<k} w[t][j] * y[t*k+j], f32 accumulation

@@ -22,7 +22,8 @@
 // W[l%32][8*(l/32)..+8] and A rows A[l%32][8*(l/32)..+8], and accumulator
 // element r of lane l is C[l%32][8*(r/4) + 4*(l/32) + r%4], four consecutive
 // output columns per register quad.  Every output element accumulates its
-// K/16 MFMA steps in increasing k, the same sequence as grouped_gemm_kernel,
+// K/16 MFMA steps in increasing k from its column's phase (k_phase; the dense
+// mode from 0), the same sequence as grouped_gemm_kernel,
 // so both kernels give identical bits.
 //
 // Epilogue: the bf16 tile goes to LDS (8-byte writes) and leaves in 16-byte
@@ -168,9 +169,13 @@ __global__ __launch_bounds__(C::THREADS) void grouped_gemm_lds_kernel(GemmArgs g
     b_src[q] = wbase + static_cast<long long>(wrow) * g.K + lchunk;
   }
 
+  const int KT = g.K / C::BK;
+  const int rot = C::BK == 64 ? k_phase<MODE>(n0, KT) : 0;
   auto issue = [&](int kt, int buf) {
     char* st = smem + buf * C::STAGE_BYTES;
-    const int koff = kt * C::BK;
+    int kr = kt + rot;
+    if (kr >= KT) kr -= KT;
+    const int koff = kr * C::BK;
 #pragma unroll
     for (int q = 0; q < C::QA; ++q) load_lds16(a_src[q] + koff, st + (wave * C::QA + q) * 1024);
 #pragma unroll
@@ -210,7 +215,6 @@ __global__ __launch_bounds__(C::THREADS) void grouped_gemm_lds_kernel(GemmArgs g
   const int wave_rows = rows - wm * C::WTM;
   const int ni_live = wave_rows <= 0 ? 0 : min(C::NI, (wave_rows + 31) >> 5);
 
-  const int KT = g.K / C::BK;
 #pragma unroll
   for (int s = 0; s < C::STAGES - 1; ++s)
     if (s < KT) issue(s, s);

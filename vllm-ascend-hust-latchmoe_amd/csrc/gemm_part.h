@@ -34,9 +34,9 @@
 // weight rows of columns outside the sub-tile load a valid row whose result
 // is dropped, so the count per stage is fixed; waves without live columns
 // skip their MFMAs, and a wave computes only its live 32-row blocks.  Every
-// output element accumulates its K/16 MFMA steps in increasing k, the order
-// of the other grouped kernels, so all of them (and both geometries) give
-// identical bits.
+// output element accumulates its K/16 MFMA steps in increasing k from its
+// column's phase (k_phase), the order of the other grouped kernels, so all of
+// them (and both geometries) give identical bits.
 //
 // Epilogue through LDS as in grouped_gemm_lds_kernel; the down tile (320 x 256
 // bf16 = 169 KB with padding) does not fit beside nothing else in 160 KB, so
@@ -122,6 +122,7 @@ __device__ __forceinline__ void part_unit(const GemmArgs& g, char* smem, int* s_
   const int fhi = lane >> 5;
   const int fsw = lds_swz<S::BK>(frow);
   const int KT = g.K / S::BK;
+  const int rot = k_phase<MODE>(n0, KT);
   const uint16_t* wbase = g.w + static_cast<long long>(slot) * g.w_slot_stride;
   if (MODE == kDown) {
     for (int t = tid; t < S::BM; t += S::THREADS)
@@ -165,7 +166,9 @@ __device__ __forceinline__ void part_unit(const GemmArgs& g, char* smem, int* s_
 
   auto issue = [&](int kt, int buf) {
     char* st = smem + buf * S::STAGE_BYTES;
-    const int koff = kt * S::BK;
+    int kr = kt + rot;
+    if (kr >= KT) kr -= KT;
+    const int koff = kr * S::BK;
 #pragma unroll
     for (int q = 0; q < S::Q_HI; ++q) {
       const int t = wave + S::NW * q;

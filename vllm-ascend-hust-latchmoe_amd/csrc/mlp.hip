@@ -18,6 +18,7 @@
 // phase_split.py:1649-1656).
 #include "gemm_lds.h"
 #include "gemm_part.h"
+#include "gemm_stream.h"
 
 namespace lmoe {
 
@@ -695,8 +696,9 @@ static void launch_combine(const uint16_t* y, const int32_t* row_idx, const uint
 }
 
 // ---------------------------------------------------------------------------
-// grouped MFMA GEMM launch (prefill).  block_m is the tile height the
-// permutation's tile table was built with: 320 runs the block-range kernel
+// grouped MFMA GEMM launch.  block_m is the tile height the permutation's
+// tile table was built with: 64 runs the weight-streaming kernel for few
+// tokens per slot (gemm_stream.h), 320 runs the block-range kernel
 // (gemm_part.h: one workgroup per CU, equal column-block shares), 256 the
 // direct-to-LDS 256 x 256 tile grid (both: K a multiple of 64, 16-byte
 // aligned operands), 128 the register-staged 128 x 128 kernel.
@@ -732,16 +734,57 @@ static bool part_offsets_fit(const GemmArgs& g, int n_pairs) {
   return a_rows * g.K <= lim && g.w_slot_stride <= lim;
 }
 
+// The wide form (two weight tiles per wave) once its blocks fill the CUs about
+// twice over at three per CU, else the narrow one, whose twice as many blocks
+// even out the last round: 128 slots of the Qwen3 shape 182 us wide against
+// 190 narrow, 64 slots at 40 tokens 123 against 113 (gate-up + down).
+constexpr long long kStreamWideBlocks = 1500;
+
+template <int MODE, bool SPLIT, bool TWO>
+static int launch_stream(const StreamArgs& a, const StreamArgs& b, int n_pairs, int max_active,
+                         hipStream_t stream) {
+  if (a.K % 64 != 0 || a.N % 64 != 0) return LMOE_ERR_SHAPE;
+  const long long tiles = n_pairs / kStreamBM + static_cast<long long>(max_active);
+  if (tiles > 65535) return LMOE_ERR_SHAPE;
+  constexpr int wide_cols = kStreamWaves * (MODE == kGateUp ? 16 : 32);
+  const int wide = (a.N + wide_cols - 1) / wide_cols;
+  if (static_cast<long long>(wide) * max_active >= kStreamWideBlocks)
+    hipLaunchKernelGGL((stream_gemm_kernel<MODE, 2, SPLIT, TWO>),
+                       dim3(wide, static_cast<unsigned>(tiles)), dim3(kStreamWaves * 64), 0, stream,
+                       a, b, n_pairs);
+  else
+    hipLaunchKernelGGL((stream_gemm_kernel<MODE, 1, SPLIT, TWO>),
+                       dim3((2 * a.N + wide_cols - 1) / wide_cols, static_cast<unsigned>(tiles)),
+                       dim3(kStreamWaves * 64), 0, stream, a, b, n_pairs);
+  return LMOE_OK;
+}
+
+// split: LMOE_PATH_STREAM
+template <int MODE, bool TWO>
+static int launch_stream(const StreamArgs& a, const StreamArgs& b, int n_pairs, int max_active,
+                         bool split, hipStream_t stream) {
+  return split ? launch_stream<MODE, true, TWO>(a, b, n_pairs, max_active, stream)
+               : launch_stream<MODE, false, TWO>(a, b, n_pairs, max_active, stream);
+}
+
 template <int MODE>
-static int launch_grouped_mfma(GemmArgs g, int n_pairs, int max_active, int block_m,
+static int launch_grouped_mfma(GemmArgs g, int n_pairs, int max_active, int block_m, int path,
                                hipStream_t stream) {
-  if (block_m != PartTile::BM && block_m != PrefillTile::BM && block_m != kBM)
+  if (path == LMOE_PATH_STREAM && block_m != kStreamBM) return LMOE_ERR_UNSUPPORTED;
+  if (block_m != PartTile::BM && block_m != PrefillTile::BM && block_m != kBM &&
+      block_m != kStreamBM)
     return LMOE_ERR_UNSUPPORTED;
   const int ub_tiles = n_pairs / block_m + max_active + 1;
   g.block_m = block_m;
   const bool aligned = ((reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.w) |
                          reinterpret_cast<uintptr_t>(g.out)) & 15u) == 0;
   if (!aligned) return LMOE_ERR_SHAPE;
+  if (block_m == kStreamBM) {
+    if (!part_offsets_fit<MODE>(g, n_pairs)) return LMOE_ERR_SHAPE;  // take block_m 256
+    const StreamArgs a{g.a, g.w, g.w_slot_stride, g.N, g.K, g.topk, g.P, g.offsets, g.sorted_pairs,
+                       g.tile_off, g.meta, static_cast<uint16_t*>(g.out)};
+    return launch_stream<MODE, false>(a, a, n_pairs, max_active, path == LMOE_PATH_STREAM, stream);
+  }
   if (block_m == PartTile::BM) {
     if (g.K % PartTile::BK != 0 || g.N % 8 != 0) return LMOE_ERR_SHAPE;
     if (!part_offsets_fit<MODE>(g, n_pairs)) return LMOE_ERR_SHAPE;  // take block_m 256
@@ -806,7 +849,7 @@ extern "C" int lmoe_gateup_silu(const void* x, int T, int H, int I, int k,
     if (st != LMOE_OK) return st;
     LMOE_RETURN_LAUNCH();
   }
-  if (path != LMOE_PATH_MFMA) return LMOE_ERR_UNSUPPORTED;
+  if (path != LMOE_PATH_MFMA && path != LMOE_PATH_STREAM) return LMOE_ERR_UNSUPPORTED;
   if (tile_off == nullptr) return LMOE_ERR_ARG;
   GemmArgs g{};
   g.topk = k;
@@ -822,7 +865,7 @@ extern "C" int lmoe_gateup_silu(const void* x, int T, int H, int I, int k,
   g.K = H;
   g.I = I;
   g.out = act;
-  st = launch_grouped_mfma<kGateUp>(g, n_pairs, max_active, block_m, stream);
+  st = launch_grouped_mfma<kGateUp>(g, n_pairs, max_active, block_m, path, stream);
   if (st != LMOE_OK) return st;
   LMOE_RETURN_LAUNCH();
 }
@@ -850,7 +893,7 @@ extern "C" int lmoe_down(const void* act, int H, int I, const void* w2_slots, in
     if (st != LMOE_OK) return st;
     LMOE_RETURN_LAUNCH();
   }
-  if (path != LMOE_PATH_MFMA) return LMOE_ERR_UNSUPPORTED;
+  if (path != LMOE_PATH_MFMA && path != LMOE_PATH_STREAM) return LMOE_ERR_UNSUPPORTED;
   if (tile_off == nullptr) return LMOE_ERR_ARG;
   GemmArgs g{};
   g.topk = 1;
@@ -865,7 +908,7 @@ extern "C" int lmoe_down(const void* act, int H, int I, const void* w2_slots, in
   g.N = H;
   g.K = I;
   g.out = yb;
-  st = launch_grouped_mfma<kDown>(g, n_pairs, max_active, block_m, stream);
+  st = launch_grouped_mfma<kDown>(g, n_pairs, max_active, block_m, path, stream);
   if (st != LMOE_OK) return st;
   LMOE_RETURN_LAUNCH();
 }
@@ -958,6 +1001,50 @@ extern "C" int lmoe_decode_mlp_two_passes(
   else LMOE_DR2N(16);
 #undef LMOE_DR2N
 #undef LMOE_DR2
+  LMOE_RETURN_LAUNCH();
+}
+
+extern "C" int lmoe_stream_mlp_two_passes(
+    const void* x, int T, int H, int I, int k, const void* w13_a, const void* w2_a, int n_slots_a,
+    const int32_t* offsets_a, const int32_t* sorted_pairs_a, const int32_t* tile_off_a,
+    const int32_t* meta_a, const void* w13_b, const void* w2_b, int n_slots_b,
+    const int32_t* offsets_b, const int32_t* sorted_pairs_b, const int32_t* tile_off_b,
+    const int32_t* meta_b, int n_pairs, int path, void* act, void* y, hipStream_t stream) {
+  int st = check_mlp_args(T, H, I, k, n_slots_a, n_pairs);
+  if (st != LMOE_OK) return st;
+  if (n_slots_b <= 0) return LMOE_ERR_ARG;
+  if (path != LMOE_PATH_MFMA && path != LMOE_PATH_STREAM) return LMOE_ERR_UNSUPPORTED;
+  if (H % 64 != 0) return LMOE_ERR_SHAPE;
+  if (n_pairs == 0) return LMOE_OK;  // an empty batch: nothing read or written
+  const void* need[] = {x, w13_a, w2_a, offsets_a, sorted_pairs_a, tile_off_a, meta_a,
+                        w13_b, w2_b, offsets_b, sorted_pairs_b, tile_off_b, meta_b, act, y};
+  for (const void* p : need)
+    if (p == nullptr) return LMOE_ERR_ARG;
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w13_a) |
+       reinterpret_cast<uintptr_t>(w13_b) | reinterpret_cast<uintptr_t>(w2_a) |
+       reinterpret_cast<uintptr_t>(w2_b) | reinterpret_cast<uintptr_t>(act) |
+       reinterpret_cast<uintptr_t>(y)) & 15u)
+    return LMOE_ERR_SHAPE;
+  const long long lim = 0x7fffffffLL;
+  if (static_cast<long long>(n_pairs) * (H > I ? H : I) > lim) return LMOE_ERR_SHAPE;
+  const int max_active = (n_pairs < n_slots_a ? n_pairs : n_slots_a) +
+                         (n_pairs < n_slots_b ? n_pairs : n_slots_b);
+  uint16_t* actb = static_cast<uint16_t*>(act);
+  uint16_t* yb = static_cast<uint16_t*>(y);
+  const uint16_t* xb = static_cast<const uint16_t*>(x);
+  const StreamArgs ga{xb, static_cast<const uint16_t*>(w13_a), slot_elems_w13(H, I), I, H, k,
+                      n_slots_a, offsets_a, sorted_pairs_a, tile_off_a, meta_a, actb};
+  const StreamArgs gb{xb, static_cast<const uint16_t*>(w13_b), slot_elems_w13(H, I), I, H, k,
+                      n_slots_b, offsets_b, sorted_pairs_b, tile_off_b, meta_b, actb};
+  const bool split = path == LMOE_PATH_STREAM;
+  st = launch_stream<kGateUp, true>(ga, gb, n_pairs, max_active, split, stream);
+  if (st != LMOE_OK) return st;
+  const StreamArgs da{actb, static_cast<const uint16_t*>(w2_a), slot_elems_w2(H, I), H, I, 1,
+                      n_slots_a, offsets_a, sorted_pairs_a, tile_off_a, meta_a, yb};
+  const StreamArgs db{actb, static_cast<const uint16_t*>(w2_b), slot_elems_w2(H, I), H, I, 1,
+                      n_slots_b, offsets_b, sorted_pairs_b, tile_off_b, meta_b, yb};
+  st = launch_stream<kDown, true>(da, db, n_pairs, max_active, split, stream);
+  if (st != LMOE_OK) return st;
   LMOE_RETURN_LAUNCH();
 }
 

@@ -4,11 +4,13 @@ fused_experts() is the body of the reference's fused-experts call with the
 slot bank in place of the expert weights: lmoe_permute remaps the top-k ids
 through log2phy and sorts the pairs by slot, then either
 
-  * lmoe_fused_moe_decode (<= 1024 pairs): gate_up GEMV + SiLU*mul, then the
-    down GEMV fused with the weighted combine (one token), or the down GEMV
-    per (row block, slot) into y and the combine (several tokens); or
-  * lmoe_grouped_mlp (GEMV or bf16 MFMA) into a flat-pair buffer y, then
-    lmoe_combine.
+  * lmoe_fused_moe_decode (a few tokens, native.layer_path): gate_up GEMV +
+    SiLU*mul, then the down GEMV fused with the weighted combine (one token),
+    or the down GEMV per (row block, slot) into y and the combine (several
+    tokens); or
+  * lmoe_grouped_mlp (bf16 MFMA: the weight-streaming kernel up to 1024
+    pairs, past them row tiles by native.prefill_block_m) into a flat-pair
+    buffer y, then lmoe_combine.
 
 Every buffer comes from a shape-keyed workspace cache, so repeated calls (and
 hipGraph replays) see the same addresses and allocate nothing.
@@ -148,25 +150,21 @@ def fused_experts(
 ) -> torch.Tensor:
     """out[t] = add[t] + sum_j w[t,j] * MLP_{slot(ids[t,j])}(x_t).
 
-    Permute, then: up to 1024 pairs (unless path is MFMA) and I <= 4096 the
-    decode body (gate_up GEMV, down GEMV fused with the combine); otherwise
-    the grouped GEMM (MFMA unless path is GEMV; always MFMA past the GEMV's
-    I <= 4096) and the combine.  topk_ids come from the caller, so a token
+    Permute, then: for a few tokens (native.layer_path) or path GEMV up to
+    1024 pairs the decode body (gate_up GEMV, down GEMV fused with the
+    combine); otherwise the grouped GEMM (path, or native.layer_path's when
+    it is AUTO) and the combine.  topk_ids come from the caller, so a token
     may name one expert twice: the decode body takes its general form,
     which holds no one-pair-per-slot assumption."""
     return _fused_experts_ws(hidden, topk_weights, topk_ids, w13_slots, w2_slots, log2phy, add=add, out=out,
                              path=path, workspace=workspace)[0]
 
 
-def _pass_path(n_pairs: int, I: int, path: int) -> int:
+def _pass_path(T: int, k: int, H: int, I: int, path: int) -> int:
     """The MLP path of one pass of a multi-pass layer, by the rule the
-    single-pass layer uses (fused_experts): the decode GEMVs up to
-    FUSED_DECODE_MAX_PAIRS pairs (and I <= GEMV_MAX_I), MFMA tiles past
-    that, so a split layer gives the unsplit layer's bits."""
-    if path != native.LMOE_PATH_AUTO:
-        return path
-    return native.LMOE_PATH_GEMV if n_pairs <= native.FUSED_DECODE_MAX_PAIRS and I <= native.GEMV_MAX_I \
-        else native.LMOE_PATH_MFMA
+    single-pass layer uses (fused_experts), so a split layer gives the
+    unsplit layer's bits."""
+    return native.layer_path(T, k, H, I) if path == native.LMOE_PATH_AUTO else path
 
 
 def _overflow_perm(hidden, k: int, overflow: PreparedSlotWeights, ws: MoEWorkspace) -> native.Permutation:
@@ -174,52 +172,63 @@ def _overflow_perm(hidden, k: int, overflow: PreparedSlotWeights, ws: MoEWorkspa
     return ws.overflow_perm(hidden.shape[0] * k, int(overflow.physical_expert_count), hidden.device)
 
 
+def _block_m(hidden, k: int, w13_slots, path: int) -> int:
+    """The row-tile height to build a pass's permutation with (the GEMVs read
+    no tile table)."""
+    if path == native.LMOE_PATH_GEMV:
+        return native.MFMA_BLOCK_M
+    if path == native.LMOE_PATH_STREAM:
+        return native.STREAM_BLOCK_M
+    T, H = hidden.shape
+    P, I = int(w13_slots.shape[0]), int(w13_slots.shape[1]) // 2
+    return native.prefill_block_m(P, H, I, hidden.device, n_pairs=T * k)
+
+
 def _overflow_permute(hidden, topk_ids, k: int, overflow: PreparedSlotWeights, ws: MoEWorkspace, *,
-                      decode: bool) -> native.Permutation:
+                      path: int) -> native.Permutation:
     """The second pass's permutation: the pairs the overflow table maps
     (every other pair is skipped).  The bank pass's row_idx then marks the
     pairs placed by either pass: the combine's row mask."""
-    T, H = hidden.shape
-    P2 = int(overflow.physical_expert_count)
-    I = int(overflow.w1.shape[1]) // 2
     perm = _overflow_perm(hidden, k, overflow, ws)
-    bm = native.MFMA_BLOCK_M if decode else native.prefill_block_m(P2, H, I, hidden.device, n_pairs=T * k)
     native.permute(topk_ids, perm, log2phy=overflow.log2phy, keep_rows=True, row_idx=ws.perm.row_idx,
-                   block_m=bm)
+                   block_m=_block_m(hidden, k, overflow.w1, path))
     return perm
 
 
-def _overflow_pass(hidden, topk_ids, k: int, overflow: PreparedSlotWeights, ws: MoEWorkspace, *, decode: bool):
+def _overflow_pass(hidden, topk_ids, k: int, overflow: PreparedSlotWeights, ws: MoEWorkspace, *, path: int):
     """Second pass of a decode step whose routed experts exceed the bank:
     the pairs the overflow table maps run from the stage buffer into their
     rows of y."""
     T = hidden.shape[0]
-    perm = _overflow_permute(hidden, topk_ids, k, overflow, ws, decode=decode)
-    native.grouped_mlp(hidden, k, overflow.w1, overflow.w2, perm, ws.act[: T * k], ws.y[: T * k],
-                       path=native.LMOE_PATH_GEMV if decode else native.LMOE_PATH_MFMA)
+    perm = _overflow_permute(hidden, topk_ids, k, overflow, ws, path=path)
+    native.grouped_mlp(hidden, k, overflow.w1, overflow.w2, perm, ws.act[: T * k], ws.y[: T * k], path=path)
 
 
-def _merged_passes(hidden, I: int, decode: bool) -> bool:
-    """Whether a decode overflow layer runs both passes' GEMVs in shared
-    launches (decode_mlp_two_passes): the decode GEMV path with rows of at
-    most TWO_PASS_MAX_COLS columns.  In the 48-layer B=64 decode graph
-    (Qwen3-30B-A3B shapes, ~33 of 48 layers with an overflow pass) shared
-    launches took the layer from 186.0 to 180.2 us, and both tables' builds
-    in one permutation launch on top of them to 176.0 us (same box)."""
-    return decode and hidden.shape[1] <= native.TWO_PASS_MAX_COLS and I <= native.TWO_PASS_MAX_COLS
+def _merged_passes(hidden, k: int, w13_slots, overflow: PreparedSlotWeights, path: int) -> bool:
+    """Whether an overflow layer runs both passes in shared launches: the
+    decode GEMV path with rows of at most TWO_PASS_MAX_COLS columns
+    (decode_mlp_two_passes), or the weight-streaming kernel in both (stream_mlp_two_passes).  In the
+    48-layer B=64 decode graph (Qwen3-30B-A3B shapes, ~33 of 48 layers with
+    an overflow pass) shared GEMV launches took the layer from 186.0 to
+    180.2 us, and both tables' builds in one permutation launch on top of
+    them to 176.0 us (same box)."""
+    if path == native.LMOE_PATH_GEMV:
+        return hidden.shape[1] <= native.TWO_PASS_MAX_COLS and \
+            int(w13_slots.shape[1]) // 2 <= native.TWO_PASS_MAX_COLS
+    return all(_block_m(hidden, k, w, path) == native.STREAM_BLOCK_M for w in (w13_slots, overflow.w1))
 
 
-def _two_passes(hidden, topk_ids, k: int, w13_slots, w2_slots, overflow: PreparedSlotWeights,
-                ws: MoEWorkspace, perm: native.Permutation | None = None) -> None:
-    """Both passes of a decode overflow layer after the bank permutation
-    (skip_unmapped): the overflow permutation (unless perm already holds
-    it), then one gate_up and one down launch serve both; y[pair] has the
-    bits of the passes run one by one."""
+def _two_passes(hidden, k: int, w13_slots, w2_slots, overflow: PreparedSlotWeights, ws: MoEWorkspace,
+                perm: native.Permutation, *, path: int) -> None:
+    """Both passes of an overflow layer, one gate_up and one down launch
+    serving both, after both permutations (the bank's with skip_unmapped);
+    y[pair] has the bits of the passes run one by one."""
     T = hidden.shape[0]
-    if perm is None:
-        perm = _overflow_permute(hidden, topk_ids, k, overflow, ws, decode=True)
-    native.decode_mlp_two_passes(hidden, k, w13_slots, w2_slots, ws.perm, overflow.w1, overflow.w2, perm,
-                                 ws.act[: T * k], ws.y[: T * k])
+    args = (hidden, k, w13_slots, w2_slots, ws.perm, overflow.w1, overflow.w2, perm, ws.act[: T * k], ws.y[: T * k])
+    if path == native.LMOE_PATH_GEMV:
+        native.decode_mlp_two_passes(*args)
+    else:
+        native.stream_mlp_two_passes(*args, path=path)
 
 
 def _fused_experts_ws(hidden, topk_weights, topk_ids, w13_slots, w2_slots, log2phy, *, add=None, out=None,
@@ -234,11 +243,13 @@ def _fused_experts_ws(hidden, topk_weights, topk_ids, w13_slots, w2_slots, log2p
     I = int(w13_slots.shape[1]) // 2
     ws = workspace or get_workspace(T, k, P, H, I, hidden.device)
     dst = out if out is not None else ws.out[:T]
-    if I > native.GEMV_MAX_I and path == native.LMOE_PATH_AUTO:
-        path = native.LMOE_PATH_MFMA
-    decode = T * k <= native.FUSED_DECODE_MAX_PAIRS and path != native.LMOE_PATH_MFMA
-    bm = native.MFMA_BLOCK_M if decode else native.prefill_block_m(P, H, I, hidden.device, n_pairs=T * k)
-    merged = overflow is not None and log2phy is not None and _merged_passes(hidden, I, decode) and not events
+    if path == native.LMOE_PATH_AUTO:
+        path = native.layer_path(T, k, H, I)
+    # the decode body; past its pair count path GEMV runs the two GEMVs apart
+    decode = path == native.LMOE_PATH_GEMV and T * k <= native.FUSED_DECODE_MAX_PAIRS
+    bm = _block_m(hidden, k, w13_slots, path)
+    merged = overflow is not None and log2phy is not None and not events and \
+        _merged_passes(hidden, k, w13_slots, overflow, path)
     if events:
         events[0].record()
     perm_b = None
@@ -249,14 +260,13 @@ def _fused_experts_ws(hidden, topk_weights, topk_ids, w13_slots, w2_slots, log2p
         native.permute(topk_ids, ws.perm, log2phy=log2phy, skip_unmapped=overflow is not None, block_m=bm)
     if overflow is not None:
         if merged:
-            _two_passes(hidden, topk_ids, k, w13_slots, w2_slots, overflow, ws, perm_b)
+            _two_passes(hidden, k, w13_slots, w2_slots, overflow, ws, perm_b, path=path)
         else:
-            mlp_path = native.LMOE_PATH_GEMV if decode else native.LMOE_PATH_MFMA
-            native.gateup_silu(hidden, k, w13_slots, ws.perm, ws.act[: T * k], path=mlp_path)
+            native.gateup_silu(hidden, k, w13_slots, ws.perm, ws.act[: T * k], path=path)
             if events:
                 events[1].record()
-            native.down(ws.act[: T * k], w2_slots, ws.perm, ws.y[: T * k], path=mlp_path)
-            _overflow_pass(hidden, topk_ids, k, overflow, ws, decode=decode)
+            native.down(ws.act[: T * k], w2_slots, ws.perm, ws.y[: T * k], path=path)
+            _overflow_pass(hidden, topk_ids, k, overflow, ws, path=path)
             if events:
                 events[2].record()
         native.combine(ws.y[: T * k], topk_weights, dst, row_mask=ws.perm.row_idx[: T * k], add=add)
@@ -333,30 +343,32 @@ def decode_layer(
         n_shared=int(spec.n_shared), w_bf16=w_out, ids=ids_out, skip_unmapped=overflow is not None,
     )
     I = int(w13_slots.shape[1]) // 2
-    decode = T * kw <= native.FUSED_DECODE_MAX_PAIRS and I <= native.GEMV_MAX_I
-    merged = overflow is not None and log2phy is not None and _merged_passes(hidden, I, decode)
+    path = native.layer_path(T, kw, int(hidden.shape[1]), I)
+    bm = _block_m(hidden, kw, w13_slots, path)
+    merged = overflow is not None and log2phy is not None and _merged_passes(hidden, kw, w13_slots, overflow, path)
     perm_b = None
-    fused_body = overflow is None and decode
+    fused_body = overflow is None and path == native.LMOE_PATH_GEMV
     if T == 1 and fused_body:
         # the one-token body reads the pairs in pair order: no sort at the
         # end of the router's chain (the same bits as the sorted form)
         w, ids, _ = native.router_gate_topk_pairs(hidden, gate_weight, logits_out, k, ws.perm, **sel)
     elif T <= ONE_LAUNCH_ROUTER_MAX_TOKENS:
-        w, ids, _ = native.router_gate_topk_permute(hidden, gate_weight, logits_out, k, ws.perm, **sel)
+        w, ids, _ = native.router_gate_topk_permute(hidden, gate_weight, logits_out, k, ws.perm, block_m=bm, **sel)
+        if merged:
+            perm_b = _overflow_permute(hidden, ids, kw, overflow, ws, path=path)
     else:
         logits = native.router_gate(hidden, gate_weight, logits_out)
         if merged:  # the overflow table's build rides with the bank's
             perm_b = _overflow_perm(hidden, kw, overflow, ws)
             sel["second"] = (perm_b, overflow.log2phy)
-        w, ids, _ = native.router_topk_permute(logits, k, ws.perm, **sel)
+        w, ids, _ = native.router_topk_permute(logits, k, ws.perm, block_m=bm, **sel)
     dst = out if out is not None else ws.out[:T]
     if overflow is not None:
         if merged:
-            _two_passes(hidden, ids, kw, w13_slots, w2_slots, overflow, ws, perm_b)
+            _two_passes(hidden, kw, w13_slots, w2_slots, overflow, ws, perm_b, path=path)
         else:
-            native.grouped_mlp(hidden, kw, w13_slots, w2_slots, ws.perm, ws.act[: T * kw], ws.y[: T * kw],
-                               path=native.LMOE_PATH_GEMV if decode else native.LMOE_PATH_MFMA)
-            _overflow_pass(hidden, ids, kw, overflow, ws, decode=decode)
+            native.grouped_mlp(hidden, kw, w13_slots, w2_slots, ws.perm, ws.act[: T * kw], ws.y[: T * kw], path=path)
+            _overflow_pass(hidden, ids, kw, overflow, ws, path=path)
         native.combine(ws.y[: T * kw], w, dst, row_mask=ws.perm.row_idx[: T * kw], add=add)
         return dst, w, ids
     if fused_body:
@@ -364,7 +376,6 @@ def decode_layer(
         native.fused_moe_decode(hidden, w, w13_slots, w2_slots, ws.perm, ws.act[: T * kw], dst, add=add,
                                 y=ws.y[: T * kw], distinct_slots=True)
     else:
-        path = native.LMOE_PATH_MFMA if I > native.GEMV_MAX_I else native.LMOE_PATH_AUTO
         native.grouped_mlp(hidden, kw, w13_slots, w2_slots, ws.perm, ws.act[: T * kw], ws.y[: T * kw], path=path)
         native.combine(ws.y[: T * kw], w, dst, row_mask=ws.perm.row_idx[: T * kw], add=add)
     return dst, w, ids
@@ -698,7 +709,7 @@ def run_wave_prefill(
                                block_m=native.prefill_block_m(len(plan.waves[w]), H, I, hidden.device, n_pairs=T * k))
                 first = False
                 native.grouped_mlp(hidden, k, prepared.w1, prepared.w2, ws.perm, ws.act[: T * k], ws.y[: T * k],
-                                   path=_pass_path(T * k, I, path))
+                                   path=_pass_path(T, k, H, I, path))
             finally:
                 runtime.end_slot_compute(handle)
             if buf is not None:
@@ -885,7 +896,7 @@ def run_device_waves(
         compute.wait_event(ready)
         native.permute(topk_ids, ws.perm, log2phy=table, skip_unmapped=True, keep_rows=w > 0, block_m=bm)
         native.grouped_mlp(hidden, k, stage.w13_slots, stage.w2_slots, ws.perm, ws.act[: T * k], ws.y[: T * k],
-                           path=_pass_path(T * k, I, path))
+                           path=_pass_path(T, k, H, I, path))
         done = torch.cuda.Event()
         done.record(compute)
         released[b] = done

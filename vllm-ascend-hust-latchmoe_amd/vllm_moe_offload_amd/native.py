@@ -25,6 +25,7 @@ LMOE_SCORING_SIGMOID = 1
 LMOE_PATH_AUTO = 0
 LMOE_PATH_GEMV = 1
 LMOE_PATH_MFMA = 2
+LMOE_PATH_STREAM = 3
 LMOE_ERR_ARG = 1000
 LMOE_ERR_SHAPE = 1001
 META_ACTIVE, META_PAIRS, META_ERRORS, META_TILES = 0, 1, 2, 3
@@ -33,6 +34,7 @@ ROUTER_SYNC_WORDS = 64 + 2 * 16 * 256  # LMOE_ROUTER_SYNC_WORDS: arrival count, 
 META_COUNT = 64  # LMOE_META_COUNT
 FLAG_UNPLACED, FLAG_ROUTER_TIMEOUT, FLAG_COUNT = 0, 1, 4  # lmoe_device_flags words
 MFMA_BLOCK_M = 256  # row-tile height of the prefill MFMA GEMM (tile table of lmoe_permute)
+STREAM_BLOCK_M = 64  # row tiles of the weight-streaming MFMA kernel (few pairs per slot)
 PART_BLOCK_M = 320  # row tiles of the one-workgroup-per-CU prefill GEMM (lmoe_grouped_mlp)
 FUSED_DECODE_MAX_PAIRS = 1024
 SKIP_KEEP_ROWS = 2  # LMOE_SKIP_KEEP_ROWS: lmoe_permute mode of the later passes of a multi-pass layer
@@ -57,6 +59,7 @@ EXPORTED_SYMBOLS = (
     "lmoe_gateup_silu",
     "lmoe_down",
     "lmoe_decode_mlp_two_passes",
+    "lmoe_stream_mlp_two_passes",
     "lmoe_combine",
     "lmoe_fused_moe_decode",
     "lmoe_fused_moe_decode_noalloc",
@@ -123,6 +126,11 @@ _SIGNATURES = {
         _i,
         [_vp, _i, _i, _i, _i, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _vp, _i, _vp,
          _vp, _vp],
+    ),
+    "lmoe_stream_mlp_two_passes": (
+        _i,
+        [_vp, _i, _i, _i, _i, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _i, _i,
+         _vp, _vp, _vp],
     ),
     "lmoe_combine": (_i, [_vp, _vp, _vp, _i, _i, _i, _vp, _vp, _vp]),
     "lmoe_fused_moe_decode": (
@@ -605,10 +613,49 @@ def _cu_count(device) -> int:
 _OFFSET32_LIMIT = 2**31 - 1
 
 
+# The decode GEMVs take a layer of up to this many tokens; past it the
+# weight-streaming MFMA kernel does.  A GEMV pays ~70 vector instructions per
+# row pair and token, the MFMA kernel has fewer bytes in flight per wave and a
+# longer chain before its first weight load.  gate-up + down, GEMV against
+# streaming (us; routing without and with the Zipf(1.1) rank bias):
+#   Qwen3 shape     16 tokens 111 / 119 and 72 / 70, 32: 159 / 171 and
+#                   102 / 94, 64: 202 / 183 and 167 / 130, 128: 280 / 197 and
+#                   257 / 169
+#   Qwen1.5-MoE     16 tokens 100 / 103 and 68 / 63, 32: 143 / 139 and
+#                   94 / 81, 48: 170 / 155 and 123 / 93
+#   DeepSeek-V3     8 tokens 712 / 718, 32: 2115 / 2099, 110: 3566 / 3134
+DECODE_GEMV_MAX_TOKENS = 32
+# Most pairs per slot, on average, of a pass on 64-row tiles: past one tile
+# per slot the second one costs as much as the wider tiles do.  Streaming
+# against the 320-row tiles (us): Qwen3 shape 600 tokens (38 pairs per slot)
+# 227 / 253, 800 tokens 250 / 259 and with the rank bias 321 / 335, 1024 (64
+# pairs) 346 / 266; Qwen1.5-MoE 400 tokens (27 pairs, skewed) 210 / 241, 800
+# (53 pairs) 277 / 252.
+STREAM_MAX_PAIRS_PER_SLOT = 40
+
+
+def layer_path(tokens: int, top_k: int, hidden: int, intermediate: int) -> int:
+    """The MLP path of a layer of `tokens` tokens with top_k pairs each: the
+    decode GEMVs for a few tokens, the streaming MFMA kernel with partial sums
+    (LMOE_PATH_STREAM, accumulation as accurate as the GEMVs') up to
+    FUSED_DECODE_MAX_PAIRS pairs, the MFMA kernels past that.  The paths round
+    differently, so the choice depends on nothing that changes when a layer is
+    split into passes (slots, waves, routing).  The streaming kernel needs
+    hidden % 64 == 0; without it the GEMVs serve all of their range."""
+    if tokens * top_k > FUSED_DECODE_MAX_PAIRS or intermediate > GEMV_MAX_I:
+        return LMOE_PATH_MFMA
+    if tokens <= DECODE_GEMV_MAX_TOKENS or hidden % 64 != 0:
+        return LMOE_PATH_GEMV
+    return LMOE_PATH_STREAM
+
+
 def prefill_block_m(n_experts: int, hidden: int, intermediate: int, device="cuda",
                     cu_count: int | None = None, n_pairs: int | None = None) -> int:
     """Row-tile height for the prefill GEMMs of one pass over n_experts slots
     (the block_m to build the permutation with).
+
+    64 selects the weight-streaming kernel, for passes of few pairs per slot
+    (n_pairs over n_experts, when n_pairs is given).
 
     320 selects the kernel with one workgroup per CU: a slot of up to 320
     pairs is one row tile, and each CU runs an equal number of units (a row
@@ -625,6 +672,8 @@ def prefill_block_m(n_experts: int, hidden: int, intermediate: int, device="cuda
         return MFMA_BLOCK_M
     if n_pairs is not None and int(n_pairs) * max(int(hidden), int(intermediate)) > _OFFSET32_LIMIT:
         return MFMA_BLOCK_M
+    if n_pairs is not None and int(n_pairs) <= STREAM_MAX_PAIRS_PER_SLOT * int(n_experts):
+        return STREAM_BLOCK_M
     cus = int(cu_count) if cu_count is not None else _cu_count(device)
     units = int(n_experts) * ((int(intermediate) + 127) // 128)
     if cus < units <= cus + cus // 4:
@@ -922,6 +971,52 @@ def decode_mlp_two_passes(
             _ptr(y), _stream(stream),
         ),
         "lmoe_decode_mlp_two_passes",
+    )
+    return y
+
+
+def stream_mlp_two_passes(
+    x: torch.Tensor,
+    top_k: int,
+    w13_a: torch.Tensor,
+    w2_a: torch.Tensor,
+    perm_a: Permutation,
+    w13_b: torch.Tensor,
+    w2_b: torch.Tensor,
+    perm_b: Permutation,
+    act: torch.Tensor,
+    y: torch.Tensor,
+    *,
+    path: int = LMOE_PATH_STREAM,
+    stream=None,
+) -> torch.Tensor:
+    """decode_mlp_two_passes on the weight-streaming MFMA kernel: y[pair] as
+    grouped_mlp(path) writes it for either pass (path STREAM or MFMA).  Both permutations hold
+    64-row tiles (block_m STREAM_BLOCK_M); the tables must map disjoint
+    experts; H % 64 == 0."""
+    lib = load_library()
+    _need(x, "x", torch.bfloat16)
+    T, H = x.shape
+    Pa, I = _check_bank(w13_a, w2_a, H)
+    Pb, Ib = _check_bank(w13_b, w2_b, H)
+    if Ib != I:
+        raise ValueError("the two passes' banks have different intermediate sizes")
+    if Pa != perm_a.n_slots or Pb != perm_b.n_slots:
+        raise ValueError("a slot bank does not match its permutation")
+    if perm_a.n_pairs != T * top_k or perm_b.n_pairs != T * top_k:
+        raise ValueError("permutations do not match T * top_k pairs")
+    if perm_a.block_m != STREAM_BLOCK_M or perm_b.block_m != STREAM_BLOCK_M:
+        raise ValueError(f"both permutations need block_m={STREAM_BLOCK_M}")
+    _need(act, "act", torch.bfloat16, (perm_a.n_pairs, I))
+    _need(y, "y", torch.bfloat16, (perm_a.n_pairs, H))
+    _check(
+        lib.lmoe_stream_mlp_two_passes(
+            _ptr(x), T, H, I, int(top_k), _ptr(w13_a), _ptr(w2_a), Pa, _ptr(perm_a.offsets),
+            _ptr(perm_a.sorted_pairs), _ptr(perm_a.tile_off), _ptr(perm_a.meta), _ptr(w13_b), _ptr(w2_b), Pb,
+            _ptr(perm_b.offsets), _ptr(perm_b.sorted_pairs), _ptr(perm_b.tile_off), _ptr(perm_b.meta),
+            perm_a.n_pairs, int(path), _ptr(act), _ptr(y), _stream(stream),
+        ),
+        "lmoe_stream_mlp_two_passes",
     )
     return y
 
