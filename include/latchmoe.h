@@ -302,11 +302,11 @@ int lmoe_gather_rows(const void* x, int H, int k, const int32_t* sorted_pairs,
  * indexed by flat pair (rows of unplaced pairs are left untouched).
  * path = LMOE_PATH_GEMV (weight-streaming, small slot groups),
  * LMOE_PATH_MFMA (bf16 MFMA tiles, block_m must equal the block_m given to
- * lmoe_permute: 64 = weight streaming for few pairs per slot, a row tile per
+ * lmoe_permute: 96 = weight streaming for few pairs per slot, a row tile per
  * workgroup, 320 = one workgroup per CU with equal shares of 32-column
  * blocks of 320-row tiles, 256 = a grid of 256 x 256 tiles, 128 = 128 x 128
- * tiles; 320 and 64 need H % 64 == 0),
- * LMOE_PATH_STREAM (the block_m 64 kernel with partial sums of 256 columns:
+ * tiles; 320 and 96 need H % 64 == 0),
+ * LMOE_PATH_STREAM (the block_m 96 kernel with partial sums of 256 columns:
  * other bits than LMOE_PATH_MFMA, accumulation as accurate as the GEMVs') or
  * LMOE_PATH_AUTO.  H % 8 == 0, I % 64 == 0.  Every block_m gives the same
  * bits. */
@@ -360,7 +360,7 @@ int lmoe_decode_mlp_two_passes(const void* x, int T, int H, int I, int k,
 
 /* lmoe_decode_mlp_two_passes on the weight-streaming MFMA kernel, for layers
  * past the GEMVs' token count: the same passes, act rows and disjoint tables,
- * tile_off in place of active, both permutations built with block_m 64.
+ * tile_off in place of active, both permutations built with block_m 96.
  * path is LMOE_PATH_MFMA or LMOE_PATH_STREAM: every value has the bits of
  * lmoe_grouped_mlp with that path over each pass.
  * H % 64 == 0, I % 64 == 0, n_pairs * max(H, I) below 2^31, every operand

@@ -1,4 +1,4 @@
-"""The weight-streaming MFMA kernel (row tiles of 64 rows): bit for bit the
+"""The weight-streaming MFMA kernel (row tiles of 96 rows): bit for bit the
 128-row tiles' act and y over the edges of its tiles, token groups, columns
 and slot table; with partial sums (path STREAM) the oracle's values, each
 token's bits whatever runs beside it, and the GEMVs' accuracy; the shared
@@ -49,15 +49,15 @@ def _run(native, d_x, k, w13, w2, d_ids, l2p, bm, n_slots, skip=False, path=None
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,I,counts", [
-    # token groups of 16: their edges, an empty slot, tiles of exactly 64 rows and of one more
-    (512, 128, [1, 15, 16, 17, 0, 31, 32, 33, 47, 48, 49, 63, 64, 65, 128, 129]),
-    (64, 64, [3, 70]),            # one K step in gate-up and in down, one block of columns
+    # token groups of 16: their edges, an empty slot, tiles of exactly 96 rows and of one more
+    (512, 128, [1, 15, 16, 17, 0, 31, 32, 33, 48, 49, 63, 64, 65, 80, 95, 96, 97, 192, 193]),
+    (64, 64, [3, 70, 100]),       # one K step in gate-up and in down, one block of columns
     (192, 192, [5, 20, 40]),      # three K steps, H and I no multiple of a block's columns
     (2048, 768, [7, 18, 36]),     # the Qwen3 expert shape
-    (320, 1408, [2, 66, 9]),      # 22 K steps in down
+    (320, 1408, [2, 90, 9]),      # 22 K steps in down
     (7168, 256, [4, 33]),         # the DeepSeek-V3 row length
-    (64, 64, [2] * 600 + [70, 0, 1]),  # past 256 and 512 slots, the wide form of the kernel in neither GEMM
-    (192, 320, [1, 17, 34] * 101),     # 303 slots of 5 column blocks: the wide form
+    (64, 64, [2] * 600 + [98, 0, 1]),  # past 256 and 512 slots, the wide form of the kernel in neither GEMM
+    (192, 320, [1, 17, 66] * 101),     # 303 slots of 5 column blocks: the wide form
 ])
 def test_stream_tiles_equal_128_row_tiles_and_oracle(H, I, counts):
     native = _native()
@@ -122,7 +122,7 @@ def test_partial_sums_round_act_as_the_gemvs_do(H, I):
 @pytest.mark.parametrize("T,k,E,Pa,Pb,H,I", [
     (64, 8, 128, 64, 64, 2048, 768),   # the batch of 64 past its 64-slot bank
     (150, 4, 40, 20, 16, 320, 192),    # guarded columns; some pairs in neither table
-    (90, 1, 4, 2, 2, 512, 64),         # slots of more than one tile in both passes
+    (400, 1, 4, 2, 2, 512, 64),        # slots of more than one tile in both passes
 ])
 def test_stream_two_passes_equal_passes_one_by_one(T, k, E, Pa, Pb, H, I):
     native = _native()

@@ -1,7 +1,7 @@
 // Weight-streaming grouped GEMM on the matrix cores, for slots of few tokens
-// (row tiles of 64 rows; wide slots are several tiles).
+// (row tiles of 96 rows; wide slots are several tiles).
 //
-// HBM bounds it: a slot of up to 64 tokens does at most 64 FLOP per weight
+// HBM bounds it: a slot of up to 96 tokens does at most 96 FLOP per weight
 // byte.  The GEMV kernels pay ~70 vector instructions per row pair and token;
 // here a token costs a column of an MFMA, so the weight stream sets the time
 // up to a few dozen tokens per slot.
@@ -34,8 +34,11 @@
 // of them, GEMV and SPLIT 1.7e-4; K 7168: 5.7e-4, 2.1e-4, 1.7e-4).
 //
 // Measured (Qwen3 shapes, 128 slots, gate-up + down): 64 tokens 182 us
-// (6.5 TB/s; GEMV 212, 320-row tiles 244), 256 tokens 200 us (245), 600
-// tokens 223 us (259); DeepSeek-V3 expert shape, 512 tokens, 3.49 ms (3.96).
+// (6.5 TB/s; GEMV 212, 320-row tiles 244), 300 tokens 207 us (247), 1024
+// tokens 245 us (269); DeepSeek-V3 expert shape, 700 tokens 3.56 ms (4.01),
+// 2048 tokens (72 per slot) 4.34 ms (4.59): there the token rows' loads and the
+// output rows' stores take the time past the weight stream's 3.4 ms, not the
+// MFMAs or LDS (a copy without most of the MFMAs: 1% less).
 #pragma once
 
 #include "gemm_mfma.h"
@@ -44,7 +47,7 @@ namespace lmoe {
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kStreamBM = 64;    // rows of a row tile (block_m of the permutation)
+constexpr int kStreamBM = 96;    // rows of a row tile (block_m of the permutation)
 constexpr int kStreamWaves = 4;  // waves per block
 constexpr int kStreamSegment = 4;  // SPLIT: stages (of 64 columns) per partial sum
 
@@ -71,12 +74,15 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // One row tile (n rows from sorted position p0, n <= 16 NG) against this
-// wave's RT tiles of weight rows, first output column n0.  live: n0 < N (a
-// wave past the last column only takes part in the barriers).
+// wave's RT tiles of weight rows, first output column n0 (the block's: nb).  A
+// wave past the last column computes the block's first columns again and
+// stores none.
 template <int MODE, int RT, bool SPLIT, int NG, int D>
-__device__ __forceinline__ void stream_tile(const StreamArgs& g, char* wlds, char* xlds, int wave,
-                                            int slot, int n0, int p0, int n, bool live) {
+__device__ __forceinline__ void stream_tile(const StreamArgs& g, char* smem, const int* rowid,
+                                            int wave, int slot, int nb, int n0, int p0, int n) {
   constexpr int NWB = kStreamWaves;
+  char* wlds = smem + wave * RT * 2048;
+  char* xlds = smem + NWB * RT * 2048;
   constexpr int XL = 2 * NG <= NWB ? 1 : 2 * NG / NWB;  // token-row loads of a wave per stage
   const int lane = threadIdx.x & 63;
   const int lr = lane >> 3, lc = lane & 7;
@@ -198,16 +204,20 @@ __device__ __forceinline__ void stream_tile(const StreamArgs& g, char* wlds, cha
 #pragma unroll
   for (int d = 0; d < D; ++d)
     if (kt + d < KT) multiply(d, kt + d);
-  if (!live) return;
   end_segment();
 
-  // lane l holds token l % 16, weight rows 4 (l / 16) .. + 3 of each tile
+  // epilogue: the block's bf16 tile to LDS, then 16-byte pieces of whole rows
+  // out (8-byte stores from the accumulators, 32 bytes per row and wave, cost
+  // the DeepSeek-V3-shaped down of 72 tokens per slot 0.3 of its 1.7 ms).
+  // Lane l holds token l % 16, weight rows 4 (l / 16) .. + 3 of each tile.
+  constexpr int COLS = MODE == kGateUp ? 8 * RT : 16 * RT;
+  constexpr int PITCH = NWB * COLS * 2 + 16;
+  constexpr int CPR = NWB * COLS / 8;  // 16-byte pieces per row
+  static_assert(16 * NG * PITCH <= NWB * RT * 2048 + 2 * NG * 2048, "the tile fits the operands' LDS");
+  lds_barrier();  // every wave is done with the operands
 #pragma unroll
   for (int q = 0; q < NG; ++q) {
-    const int tk = q * 16 + r16;
-    const bool in = tk < n;
-    const int pos = p0 + (in ? tk : 0);
-    uint16_t* dst = g.out + static_cast<long long>(MODE == kGateUp ? pos : g.sorted_pairs[pos]) * g.N;
+    char* row = smem + (q * 16 + r16) * PITCH + wave * COLS * 2;
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
       const f32x4_t v = SPLIT ? sum[SPLIT ? t : 0][SPLIT ? q : 0] : acc[t][q];
@@ -218,15 +228,23 @@ __device__ __forceinline__ void stream_tile(const StreamArgs& g, char* wlds, cha
           gv[e] = uv[e] = v[e];
           permlane_swap<32>(gv[e], uv[e]);  // lanes < 32: own gate values, lane + 32's up values
         }
-        if (in && lane < 32)
-          *reinterpret_cast<uint2*>(dst + n0 + 8 * t + 4 * kg) =
+        if (lane < 32)
+          *reinterpret_cast<uint2*>(row + t * 16 + kg * 8) =
               make_uint2(swiglu_bf16x2(gv[0], uv[0], gv[1], uv[1]),
                          swiglu_bf16x2(gv[2], uv[2], gv[3], uv[3]));
-      } else if (in) {
-        *reinterpret_cast<uint2*>(dst + n0 + 16 * t + 4 * kg) =
+      } else {
+        *reinterpret_cast<uint2*>(row + t * 32 + kg * 8) =
             make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
       }
     }
+  }
+  lds_barrier();
+  for (int e = threadIdx.x; e < n * CPR; e += NWB * 64) {
+    const int r = e / CPR, c = e % CPR;
+    if (nb + 8 * c >= g.N) continue;  // columns of waves past the last one
+    const long long dst = MODE == kGateUp ? p0 + r : rowid[r];
+    *reinterpret_cast<uint4*>(g.out + dst * g.N + nb + 8 * c) =
+        *reinterpret_cast<const uint4*>(smem + r * PITCH + c * 16);
   }
 }
 
@@ -254,13 +272,14 @@ __device__ __forceinline__ int stream_tile_slot(const int32_t* tile_off, int P, 
 // passes of a decode layer past its bank in one launch, the tiles of g first,
 // then those of g2, whose act rows follow the pairs g places (an overflow
 // slot's rows stay inside the n_pairs rows of the act buffer).  Registers:
-// RT 1 leaves 4 waves per SIMD, RT 2 three, with the partial sums two (two or
-// three waves take the same time).
+// RT 1 leaves 4 waves per SIMD, RT 2 three, with the partial sums three and two
+// (two or three waves take the same time).
 template <int MODE, int RT, bool SPLIT, bool TWO>
-__global__ __launch_bounds__(kStreamWaves * 64, RT == 1 ? 4 : SPLIT ? 2 : 3) void stream_gemm_kernel(
+__global__ __launch_bounds__(kStreamWaves * 64, RT == 2 && SPLIT ? 2 : RT == 1 && !SPLIT ? 4 : 3) void stream_gemm_kernel(
     StreamArgs g, StreamArgs g2, int n_pairs) {
   __shared__ __attribute__((aligned(1024))) char
       smem[kStreamWaves * RT * 2048 + 2 * (kStreamBM / 16) * 2048];
+  __shared__ int rowid[kStreamBM];
   int tile = blockIdx.y;
   const int tiles = g.meta[LMOE_META_TILES];
   bool second = false;
@@ -283,15 +302,16 @@ __global__ __launch_bounds__(kStreamWaves * 64, RT == 1 ? 4 : SPLIT ? 2 : 3) voi
   int n = min(kStreamBM, g.offsets[slot + 1] - p0);
   if (TWO && second) n = min(n, n_pairs - base - p0);
   if (n <= 0) return;  // uniform over the block
+  // destination rows, read here once: in the store loop each would be a
+  // load's latency
+  if (MODE == kDown && threadIdx.x < n) rowid[threadIdx.x] = g.sorted_pairs[p0 + threadIdx.x];
   constexpr int COLS = MODE == kGateUp ? 8 * RT : 16 * RT;  // output columns of a wave
-  int n0 = (blockIdx.x * kStreamWaves + wave) * COLS;
-  const bool live = n0 < g.N;
-  if (!live) n0 = blockIdx.x * kStreamWaves * COLS;
-  char* wlds = smem + wave * RT * 2048;
-  char* xlds = smem + kStreamWaves * RT * 2048;
-  if (n <= 16) stream_tile<MODE, RT, SPLIT, 1, 4>(g, wlds, xlds, wave, slot, n0, p0, n, live);
-  else if (n <= 32) stream_tile<MODE, RT, SPLIT, 2, 4>(g, wlds, xlds, wave, slot, n0, p0, n, live);
-  else stream_tile<MODE, RT, SPLIT, 4, RT == 2 || SPLIT ? 2 : 3>(g, wlds, xlds, wave, slot, n0, p0, n, live);
+  const int nb = blockIdx.x * kStreamWaves * COLS;
+  const int n0 = nb + wave * COLS < g.N ? nb + wave * COLS : nb;
+  if (n <= 16) stream_tile<MODE, RT, SPLIT, 1, 4>(g, smem, rowid, wave, slot, nb, n0, p0, n);
+  else if (n <= 32) stream_tile<MODE, RT, SPLIT, 2, 4>(g, smem, rowid, wave, slot, nb, n0, p0, n);
+  else if (n <= 64) stream_tile<MODE, RT, SPLIT, 4, 2>(g, smem, rowid, wave, slot, nb, n0, p0, n);
+  else stream_tile<MODE, RT, SPLIT, 6, 2>(g, smem, rowid, wave, slot, nb, n0, p0, n);
 }
 
 }  // namespace lmoe

@@ -697,7 +697,7 @@ static void launch_combine(const uint16_t* y, const int32_t* row_idx, const uint
 
 // ---------------------------------------------------------------------------
 // grouped MFMA GEMM launch.  block_m is the tile height the permutation's
-// tile table was built with: 64 runs the weight-streaming kernel for few
+// tile table was built with: 96 runs the weight-streaming kernel for few
 // tokens per slot (gemm_stream.h), 320 runs the block-range kernel
 // (gemm_part.h: one workgroup per CU, equal column-block shares), 256 the
 // direct-to-LDS 256 x 256 tile grid (both: K a multiple of 64, 16-byte

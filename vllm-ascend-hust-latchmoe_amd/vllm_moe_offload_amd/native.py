@@ -34,7 +34,7 @@ ROUTER_SYNC_WORDS = 64 + 2 * 16 * 256  # LMOE_ROUTER_SYNC_WORDS: arrival count, 
 META_COUNT = 64  # LMOE_META_COUNT
 FLAG_UNPLACED, FLAG_ROUTER_TIMEOUT, FLAG_COUNT = 0, 1, 4  # lmoe_device_flags words
 MFMA_BLOCK_M = 256  # row-tile height of the prefill MFMA GEMM (tile table of lmoe_permute)
-STREAM_BLOCK_M = 64  # row tiles of the weight-streaming MFMA kernel (few pairs per slot)
+STREAM_BLOCK_M = 96  # row tiles of the weight-streaming MFMA kernel (few pairs per slot)
 PART_BLOCK_M = 320  # row tiles of the one-workgroup-per-CU prefill GEMM (lmoe_grouped_mlp)
 FUSED_DECODE_MAX_PAIRS = 1024
 SKIP_KEEP_ROWS = 2  # LMOE_SKIP_KEEP_ROWS: lmoe_permute mode of the later passes of a multi-pass layer
@@ -625,13 +625,14 @@ _OFFSET32_LIMIT = 2**31 - 1
 #                   94 / 81, 48: 170 / 155 and 123 / 93
 #   DeepSeek-V3     8 tokens 712 / 718, 32: 2115 / 2099, 110: 3566 / 3134
 DECODE_GEMV_MAX_TOKENS = 32
-# Most pairs per slot, on average, of a pass on 64-row tiles: past one tile
-# per slot the second one costs as much as the wider tiles do.  Streaming
-# against the 320-row tiles (us): Qwen3 shape 600 tokens (38 pairs per slot)
-# 227 / 253, 800 tokens 250 / 259 and with the rank bias 321 / 335, 1024 (64
-# pairs) 346 / 266; Qwen1.5-MoE 400 tokens (27 pairs, skewed) 210 / 241, 800
-# (53 pairs) 277 / 252.
-STREAM_MAX_PAIRS_PER_SLOT = 40
+# Most pairs per slot, on average, of a pass on STREAM_BLOCK_M-row tiles: past
+# one tile per slot the second one costs as much as the wider tiles do.
+# Streaming against the 320-row tiles (us): Qwen3 shape 1024 tokens (64 pairs
+# per slot) 245 / 269, 1300 (81) 272 / 274, 1600 (100) 400 / 285, with half the
+# rank bias 800 tokens 269 / 317, 1300 330 / 341; Qwen1.5-MoE, the same bias,
+# 400 tokens (27 pairs) 210 / 246, 800 (53) 267 / 258; DeepSeek-V3 shape 1024
+# tokens (36 pairs) 3734 / 4127, 2048 (72) 4341 / 4590.
+STREAM_MAX_PAIRS_PER_SLOT = 75
 
 
 def layer_path(tokens: int, top_k: int, hidden: int, intermediate: int) -> int:
@@ -654,7 +655,7 @@ def prefill_block_m(n_experts: int, hidden: int, intermediate: int, device="cuda
     """Row-tile height for the prefill GEMMs of one pass over n_experts slots
     (the block_m to build the permutation with).
 
-    64 selects the weight-streaming kernel, for passes of few pairs per slot
+    STREAM_BLOCK_M selects the weight-streaming kernel, for passes of few pairs per slot
     (n_pairs over n_experts, when n_pairs is given).
 
     320 selects the kernel with one workgroup per CU: a slot of up to 320
@@ -991,8 +992,8 @@ def stream_mlp_two_passes(
     stream=None,
 ) -> torch.Tensor:
     """decode_mlp_two_passes on the weight-streaming MFMA kernel: y[pair] as
-    grouped_mlp(path) writes it for either pass (path STREAM or MFMA).  Both permutations hold
-    64-row tiles (block_m STREAM_BLOCK_M); the tables must map disjoint
+    grouped_mlp(path) writes it for either pass (path STREAM or MFMA).  Both
+    permutations are built with block_m STREAM_BLOCK_M; the tables must map disjoint
     experts; H % 64 == 0."""
     lib = load_library()
     _need(x, "x", torch.bfloat16)
