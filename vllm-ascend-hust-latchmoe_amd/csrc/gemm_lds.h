@@ -79,6 +79,7 @@ struct LdsTile {
   static constexpr int MAIN_BYTES = RING_BYTES > OUT_BYTES ? RING_BYTES : OUT_BYTES;
   static constexpr int LDS_BYTES = MAIN_BYTES + BM * 4;  // + destination row ids
   static_assert(STAGES >= 2 && LDS_BYTES <= 160 * 1024, "LDS footprint too large");
+  static_assert((STAGES - 2) * Q < 64, "the wait counts at most 63 loads");
 };
 
 // Wait until at most N of this wave's vector-memory loads are in flight (and
@@ -88,6 +89,17 @@ struct LdsTile {
 template <int N>
 __device__ __forceinline__ void vm_wait_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// vm_wait_barrier with at most min(ahead, MAX) stages of Q loads in flight
+template <int Q, int MAX>
+__device__ __forceinline__ void wait_stages(int ahead) {
+  if constexpr (MAX > 0) {
+    if (ahead >= MAX) vm_wait_barrier<MAX * Q>();
+    else wait_stages<Q, MAX - 1>(ahead);
+  } else {
+    vm_wait_barrier<0>();
+  }
 }
 
 __device__ __forceinline__ void load_lds16(const uint16_t* src, char* lds) {
@@ -228,10 +240,7 @@ __global__ __launch_bounds__(C::THREADS) void grouped_gemm_lds_kernel(GemmArgs g
     for (int kt = 0; kt < KT; ++kt) {
       // stage kt landed (loads of the later stages may stay in flight) and
       // every wave is done with the buffer the next issue overwrites
-      const int ahead = KT - 1 - kt;
-      if (C::STAGES >= 4 && ahead >= 2) vm_wait_barrier<(C::STAGES >= 4 ? 2 : 0) * C::Q>();
-      else if (C::STAGES >= 3 && ahead >= 1) vm_wait_barrier<(C::STAGES >= 3 ? 1 : 0) * C::Q>();
-      else vm_wait_barrier<0>();
+      wait_stages<C::Q, C::STAGES - 2>(KT - 1 - kt);
       if (kt + C::STAGES - 1 < KT) {
         int nb = buf + C::STAGES - 1;
         if (nb >= C::STAGES) nb -= C::STAGES;
@@ -348,11 +357,6 @@ __global__ __launch_bounds__(C::THREADS) void grouped_gemm_lds_kernel(GemmArgs g
     *reinterpret_cast<uint4*>(dst) = v;
   }
 }
-
-// 64-row x 128-column tiles with four stages of operands in flight: for a
-// few dozen tiles whose time is the K chain (the router gate over many
-// tokens)
-using SmallTile = LdsTile<64, 128, 1, 2, 4>;
 
 // Upper bound on launched workgroups for up to ub_tiles row tiles: the grid
 // is a multiple of 8 with ceil(items / 8) workgroups per XCD.

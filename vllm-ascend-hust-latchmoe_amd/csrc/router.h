@@ -22,8 +22,18 @@ constexpr int kGateShortChunks = 4;  // the one-launch router's short-row gate: 
 // threads of every one-token one-launch router: the gate form's eight gate
 // rows per block, which also covers the slot scan up to kMaxSlots / 16
 constexpr int kOneTokenRouterThreads = 512;
-// router gate at large T: 64-row x 128-expert tiles, 2 waves, 4-stage ring
-using DenseGateTile = SmallTile;
+// Router gate at large T (grouped_gemm_lds_kernel<kDense>).  A tile is one
+// chain over K whose stages, about 0.25 us per 64 columns however small the
+// tile, set the time, so while the tiles are at most one per CU a tile is
+// 64 x 64, a 32 x 32 block for each of four waves: 65 to 4096 tokens x 2048 x 128
+// experts 11 us (19 with 64 x 128 tiles of two waves), 8192 tokens 12.4
+// (19.7), 65 to 2048 tokens x 7168 x 256 experts 31 us (57).  Past one per
+// CU the 64 x 128 tiles, which read the operands less often, are as fast or
+// faster: 16384 tokens x 2048 x 128 experts 21.0 us against 22.8, 8192 x
+// 7168 x 256 58 against 63.
+using DenseGateTile = LdsTile<64, 64, 2, 2, 6>;
+using DenseGateWideTile = LdsTile<64, 128, 1, 2, 4>;
+constexpr int kDenseGateTiles = 256;  // tiles of one round of the CUs
 constexpr int kGateTok = 4;         // tokens per reduction in the gate GEMV
 // one-launch router: tagged logit words from int32 offset 64 of sync (256
 // bytes past the arrival counter), and the re-reads of a stale word

@@ -68,10 +68,7 @@ extern "C" int lmoe_router_gate(const void* x, const void* wg, int T, int H,
   if (T > 64 && H % DenseGateTile::BK == 0 && E % 8 == 0 &&
       ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(wg) |
         reinterpret_cast<uintptr_t>(logits)) & 15u) == 0) {
-    // large token counts: one dense bf16 MFMA GEMM, logits = x . wg^T, with
-    // 64 x 128 tiles and four stages of operands in flight per workgroup
-    // (a few dozen tiles, each a long K chain: the chain's stages, not the
-    // tile count, set the time)
+    // large token counts: one dense bf16 MFMA GEMM, logits = x . wg^T
     GemmArgs g{};
     g.a = static_cast<const uint16_t*>(x);
     g.w = static_cast<const uint16_t*>(wg);
@@ -81,10 +78,17 @@ extern "C" int lmoe_router_gate(const void* x, const void* wg, int T, int H,
     g.M_dense = T;
     g.out = logits;
     g.out_f32 = logits_f32;
-    const int grid = lds_gemm_grid((T + DenseGateTile::BM - 1) / DenseGateTile::BM,
-                                   (E + DenseGateTile::BN - 1) / DenseGateTile::BN);
-    hipLaunchKernelGGL((grouped_gemm_lds_kernel<kDense, DenseGateTile>), dim3(grid),
-                       dim3(DenseGateTile::THREADS), 0, stream, g);
+    const auto tiles = [&](auto tile) {
+      using C = decltype(tile);
+      return lds_gemm_grid((T + C::BM - 1) / C::BM, (E + C::BN - 1) / C::BN);
+    };
+    if (tiles(DenseGateTile{}) <= kDenseGateTiles)
+      hipLaunchKernelGGL((grouped_gemm_lds_kernel<kDense, DenseGateTile>),
+                         dim3(tiles(DenseGateTile{})), dim3(DenseGateTile::THREADS), 0, stream, g);
+    else
+      hipLaunchKernelGGL((grouped_gemm_lds_kernel<kDense, DenseGateWideTile>),
+                         dim3(tiles(DenseGateWideTile{})), dim3(DenseGateWideTile::THREADS), 0,
+                         stream, g);
     LMOE_RETURN_LAUNCH();
   }
   if (T > 64) {
