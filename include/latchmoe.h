@@ -398,13 +398,18 @@ int lmoe_down_combine(const void* act, int T, int H, int I, int k,
 
 /* Decode MoE for small pair counts:
  *   out[t] = (add ? add[t] : 0) + sum_j w[t][j] * W2_s(t,j) act[pos(t,j)].
- * gate_up GEMV + SiLU*mul into act (sorted order), then either the down GEMV
- * fused with the weighted combine (each workgroup owns a few output columns
- * of every token; two launches, used for T*k <= 16 or y == NULL), or, for
- * more pairs with a y workspace ([T*k, H] bf16, flat pair order on return),
- * the down GEMV per (row block, slot) into y and the combine (three
- * launches: no workgroup walks the slots in turn).  Both give the same out
- * bit for bit.  Each slot's weights are read once however many tokens chose
+ * gate_up GEMV + SiLU*mul into act (sorted order), then one of three forms of
+ * the rest, which give the same out bit for bit:
+ *   the down GEMV fused with the weighted combine, every workgroup walking the
+ *   slots for a few output columns of every token (T*k <= 16, or y == NULL);
+ *   for 2 and more tokens of up to 256 pairs with 256 < I <= 1024 and
+ *   1792 <= H <= 2048 or 896 <= H <= 1024 (one workgroup per CU), the same in
+ *   a form that streams the slots' rows without a gap;
+ *   for more than 16 pairs with a y workspace, else, the down GEMV per (row
+ *   block, slot) into y and the combine (three launches).
+ * With more than 16 pairs y, where given, holds the [T*k, H] bf16 down rows in
+ * flat pair order on return.  Each slot's weights are read once however many
+ * tokens chose
  * it.  distinct_slots != 0 promises that no slot serves two pairs of one
  * token (true for ids from the routers, which pick distinct experts, through
  * a slot table, which maps distinct experts to distinct slots); with one

@@ -4,8 +4,8 @@
 // row is read from HBM exactly once with 16-byte non-temporal loads, all of a
 // wave's rows in flight at once; token rows and act rows come from L2.  The
 // down projection is fused with the weighted combine (one workgroup owns R
-// output columns for every token), so the decode layer body is permute + two
-// kernels.  (A single launch would need a cross-block hand-off of act; the
+// output columns for every token) where the slots serve a pair each or H gives
+// a workgroup to every CU, so the decode layer body is permute + two kernels.  (A single launch would need a cross-block hand-off of act; the
 // agent-scope fences that takes write back / invalidate a whole XCD L2 each
 // and cost far more than a kernel boundary, which in a captured graph is
 // back to back.)
@@ -433,6 +433,149 @@ __global__ __launch_bounds__(256) void down_combine_gemv_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// down GEMV + weighted combine for a few tokens (n_pairs <= kFewPairs), every
+// slot's pairs in one launch: no second kernel that reads y back.  grid ceil(H / (2 RH)):
+// a block owns 2 RH output columns for every active slot, its waves take the
+// slots in list order (heavy slots first) as they become free.  Half wave h
+// holds rows RH h .. RH h + RH - 1 of the slot's W2 block (DNC 16-byte chunks
+// per lane and row, non-temporal; one contiguous piece of 2 RH rows per slot).
+// Order of a wave's loads: the slot's first act rows, then the next slot's W2
+// rows, so that waiting for the former leaves the latter in flight.  y (bf16
+// values) stays in LDS; the block combines its columns of every token in pair
+// order and, where the caller gave a y, stores it there too.  Every value is formed as in down_rows_kernel and combine_kernel: the
+// same bits.
+// ---------------------------------------------------------------------------
+constexpr int kFewPairs = 256;
+constexpr int kFewWaves = 8;
+
+template <int DNC, int RH, bool FULL>
+__global__ __launch_bounds__(kFewWaves * 64) void down_combine_few_kernel(
+    const uint16_t* __restrict__ act, int I, int H, int T, int topk,
+    const uint16_t* __restrict__ w2, const int32_t* __restrict__ offsets,
+    const int32_t* __restrict__ active, int P, const int32_t* __restrict__ row_idx,
+    const uint16_t* __restrict__ wts, const uint16_t* __restrict__ add,
+    uint16_t* __restrict__ y, uint16_t* __restrict__ out) {
+  constexpr int NW = kFewWaves;
+  constexpr int R = 2 * RH;
+  constexpr int LV = RH == 4 ? 2 : 1;
+  constexpr int QB = DNC <= 3 ? 4 : 2;  // pairs per step
+  __shared__ float s_y[kFewPairs * R];
+  __shared__ int s_pos[kFewPairs];
+  __shared__ float s_w[kFewPairs];
+  __shared__ int s_next;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l5 = lane & 31;
+  const int half = lane >> 5;
+  const int h0 = blockIdx.x * R + half * RH;
+  const int NP = T * topk;
+
+  uint4 w[2][RH][DNC];
+  auto load_rows = [&](int s, int b) {
+    const uint16_t* base = w2 + static_cast<size_t>(s) * H * I;
+#pragma unroll
+    for (int r = 0; r < RH; ++r)
+#pragma unroll
+      for (int c = 0; c < DNC; ++c) {
+        const int col = c * 256 + l5 * 8;
+        w[b][r][c] = load_stream16_g<!FULL>(base, (h0 + r) * I + col, col < I);
+      }
+  };
+  // the waves' first slots are ranks 0 .. NW - 1, the rest by the counter
+  auto slot_at = [&](int rank) {
+    return __builtin_amdgcn_readfirstlane(rank < P ? active[rank] : -1);
+  };
+  auto next_rank = [&]() {
+    int v = 0;
+    if (lane == 0) v = atomicAdd(&s_next, 1);
+    return __builtin_amdgcn_readfirstlane(v);
+  };
+  int cur = slot_at(wave);
+  if (cur >= 0) load_rows(cur, 0);
+  if (tid == 0) s_next = NW;
+  for (int p = tid; p < NP; p += NW * 64) {
+    const int pos = row_idx[p];
+    s_pos[p] = pos;
+    s_w[p] = bf16_to_f32(wts[p]);
+    if (blockIdx.x == 0 && pos < 0) add_device_flag(LMOE_FLAG_UNPLACED, 1);
+  }
+  __syncthreads();
+
+  auto serve = [&](int b) {  // slot cur from w[b]; on return cur is the next slot, loading into w[1 - b]
+    const int p0 = offsets[cur];
+    const int n = offsets[cur + 1] - p0;
+    const int nxt = slot_at(next_rank());
+    for (int q0 = 0; q0 < n; q0 += QB) {
+      uint4 a[QB][DNC];
+#pragma unroll
+      for (int q = 0; q < QB; ++q) {
+        const uint16_t* ar = act + static_cast<size_t>(p0 + min(q0 + q, n - 1)) * I;
+#pragma unroll
+        for (int c = 0; c < DNC; ++c) {
+          const int col = c * 256 + l5 * 8;
+          a[q][c] = load16_g<!FULL>(ar, col, col < I);
+        }
+      }
+      if (q0 == 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (nxt >= 0) load_rows(nxt, 1 - b);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int q = 0; q < QB; ++q) {
+        if (q0 + q >= n) break;  // uniform
+        float v[RH];
+#pragma unroll
+        for (int r = 0; r < RH; ++r) v[r] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < DNC; ++c)
+#pragma unroll
+          for (int r = 0; r < RH; ++r) v[r] = dot8(a[q][c], w[b][r][c], v[r]);
+        const float tot = reduce_scatter<RH, 4, 0>(v, lane);
+        const int r = scatter_index<4, 0, LV>(lane);
+        if ((l5 & ((1 << (5 - LV)) - 1)) == 0)
+          s_y[(p0 + q0 + q) * R + half * RH + r] = round_bf16(tot);  // GMM2 output is bf16
+      }
+    }
+    cur = nxt;
+  };
+  while (cur >= 0) {
+    serve(0);
+    if (cur < 0) break;
+    serve(1);
+  }
+  __syncthreads();
+  for (int e = tid; e < T * R; e += NW * 64) {
+    const int t = e / R, r = e % R;
+    const int h = blockIdx.x * R + r;
+    float acc = 0.0f;
+    for (int j = 0; j < topk; ++j) {
+      const int pos = s_pos[t * topk + j];
+      if (pos >= 0) acc += s_w[t * topk + j] * s_y[pos * R + r];
+    }
+    if (add != nullptr) acc += bf16_to_f32(add[static_cast<size_t>(t) * H + h]);
+    out[static_cast<size_t>(t) * H + h] = static_cast<uint16_t>(f32_to_bf16_bits(acc));
+  }
+  if (y != nullptr) {
+    for (int p = tid; p < NP; p += NW * 64) {
+      const int pos = s_pos[p];
+      if (pos < 0) continue;  // a pair no pass placed: its y row stays as it is
+      uint32_t v[R / 2];
+#pragma unroll
+      for (int r = 0; r < R; r += 2)  // s_y holds bf16 values: their upper halves
+        v[r / 2] = (__float_as_uint(s_y[pos * R + r]) >> 16) |
+                   (__float_as_uint(s_y[pos * R + r + 1]) & 0xffff0000u);
+      uint16_t* yp = y + static_cast<size_t>(p) * H + blockIdx.x * R;
+      if constexpr (R == 8)
+        *reinterpret_cast<uint4*>(yp) = make_uint4(v[0], v[1], v[2], v[3]);
+      else
+        *reinterpret_cast<uint2*>(yp) = make_uint2(v[0], v[1]);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // down GEMV per (row block, slot), y in bf16.  grid (ceil(H / (8 R)),
 // max_active); half wave hw of block (bx, a) owns rows h0 = (8 bx + hw) R ..
 // h0 + R - 1 of the a-th active slot: DNC 16-byte chunks per lane and row
@@ -687,6 +830,49 @@ static int launch_down_rows(const uint16_t* act, int H, int I, const uint16_t* w
 #undef LMOE_DR
 #undef LMOE_DR1
   return LMOE_OK;
+}
+
+// down_combine_few_kernel serves 2 and more tokens of up to kFewPairs pairs
+// where 8 or (H <= 1024) 4 output columns per block make one block for nearly
+// every CU (224 to 256 of them): its waves stream a CU's whole share of W2
+// from start to end; bound by the weights' stream.  Decode body, separate
+// kernels -> this one (us, 2 / 8 / 32 tokens; y given, its store is up to 1 us):
+//   128 experts, top 8, H 2048, I 768   26.8 / 52.6 / 103.9 -> 24.7 / 50.8 / 102.2
+//   16 experts, top 2, H 2048, I 1024   15.3 / 23.2 / 42.7 -> 13.8 / 20.4 / 40.7
+//   64 experts, top 8, H 1024, I 768    19.5 / 31.0 / 57.5 -> 17.7 / 29.0 / 56.3
+// Where the line lies: several blocks per CU run one after another without
+// overlap (H 7168, I 704, 16 tokens 138 -> 147); CUs without a block lose more
+// than the launch saved (H 1536, I 704: 192 blocks, 8 tokens 43.8 -> 45.9);
+// I <= 256 leaves half of each wave idle (H 1024, 32 tokens 33.8 -> 36.1); and
+// I > 1024 needs two rows per half wave (I 1408, 24 tokens 87 -> 98).
+static bool down_combine_few_fits(int T, int n_pairs, int H, int I) {
+  const int blocks = H <= 1024 ? (H + 3) / 4 : (H + 7) / 8;
+  return T > 1 && n_pairs <= kFewPairs && I > 256 && I <= 1024 && blocks >= 224 && blocks <= 256;
+}
+
+static void launch_down_combine_few(const uint16_t* act, int T, int H, int I, int k,
+                                    const uint16_t* w2, int n_slots, const uint16_t* w,
+                                    const int32_t* offsets, const int32_t* row_idx,
+                                    const int32_t* active, const uint16_t* add, uint16_t* y,
+                                    uint16_t* out, hipStream_t stream) {
+#define LMOE_DF1(DNC, RH, FULL)                                                                   \
+  hipLaunchKernelGGL((down_combine_few_kernel<DNC, RH, FULL>), dim3((H + 2 * (RH)-1) / (2 * (RH))), \
+                     dim3(kFewWaves * 64), 0, stream, act, I, H, T, k, w2, offsets, active,       \
+                     n_slots, row_idx, w, add, y, out)
+#define LMOE_DF(DNC)                                                             \
+  do {                                                                           \
+    const bool full = I == (DNC)*256; /* H % 8 == 0: no row is past H */         \
+    if (H <= 1024 && full) LMOE_DF1(DNC, 2, true);                               \
+    else if (H <= 1024) LMOE_DF1(DNC, 2, false);                                 \
+    else if (full) LMOE_DF1(DNC, 4, true);                                       \
+    else LMOE_DF1(DNC, 4, false);                                                \
+  } while (0)
+  const int dnc = (I + 255) / 256;
+  if (dnc <= 2) LMOE_DF(2);
+  else if (dnc <= 3) LMOE_DF(3);
+  else LMOE_DF(4);
+#undef LMOE_DF
+#undef LMOE_DF1
 }
 
 static void launch_combine(const uint16_t* y, const int32_t* row_idx, const uint16_t* w, int T,
@@ -1141,12 +1327,21 @@ extern "C" int lmoe_fused_moe_decode(const void* x, int T, int H, int I, int k,
                               sorted_pairs, active, meta, max_active, one, n_pairs,
                               static_cast<uint16_t*>(act), stream);
   if (st != LMOE_OK) return st;
+  if (down_combine_few_fits(T, n_pairs, H, I)) {
+    launch_down_combine_few(static_cast<const uint16_t*>(act), T, H, I, k,
+                            static_cast<const uint16_t*>(w2_slots), n_slots, w, offsets, row_idx,
+                            active, static_cast<const uint16_t*>(add),
+                            n_pairs > 16 ? static_cast<uint16_t*>(y) : nullptr,
+                            static_cast<uint16_t*>(out), stream);
+    LMOE_RETURN_LAUNCH();
+  }
   if (y != nullptr && T > 1 && n_pairs > 16) {
     // slots serving several tokens: down per (row block, slot) into y (flat
     // pair order), then the combine.  Up to 16 pairs (two slots per half
-    // wave of the fused kernel) the fused down + combine is faster: 27.7
-    // against 28.9 us per layer at 2 tokens, equal at 4, slower from 8 on;
-    // both give the same bits.
+    // wave of the fused kernel) the fused down + combine is faster (Qwen3
+    // shape, before that shape had a form of its own: 27.7 against 28.9 us
+    // per layer at 2 tokens, equal at 4, slower from 8 on); both give the
+    // same bits.
     st = launch_down_rows(static_cast<const uint16_t*>(act), H, I,
                           static_cast<const uint16_t*>(w2_slots), offsets, sorted_pairs, active,
                           max_active, static_cast<uint16_t*>(y), stream);

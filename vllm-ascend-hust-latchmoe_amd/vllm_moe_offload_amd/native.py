@@ -1067,9 +1067,9 @@ def fused_moe_decode(
     stream=None,
 ) -> torch.Tensor:
     """Decode layer body: gate_up GEMV, then down GEMV fused with the combine
-    (up to 16 pairs, or no y), or with a [T*k, H] bf16 workspace y and more
-    pairs the down GEMV per (row block, slot) into y and the combine; same out
-    either way.  distinct_slots: the caller promises that no slot serves two
+    (up to 16 pairs, no y, or up to 256 pairs where H gives about one workgroup
+    per CU), or with a [T*k, H] bf16 workspace y and more pairs the down GEMV
+    per (row block, slot) into y and the combine; same out either way.  distinct_slots: the caller promises that no slot serves two
     pairs of one token (router-fed ids through a slot table); with one token
     it selects the faster one-pair-per-slot kernels."""
     lib = load_library()
