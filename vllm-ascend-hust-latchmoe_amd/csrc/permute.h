@@ -124,15 +124,17 @@ __device__ __forceinline__ bool heavy_slot(int count, int placed) {
 }
 
 // Order key of a heavy slot: a larger key is listed first (higher count,
-// then lower slot); never 0, the value of an empty entry of a key list.
-__device__ __forceinline__ uint64_t heavy_key(int count, int s) {
-  return (static_cast<uint64_t>(count) << 32) | (0xffffffffu - static_cast<uint32_t>(s));
-}
-
-// The same order in 32 bits, for count < 65536 and s < 65536.
-__device__ __forceinline__ uint32_t heavy_key16(int count, int s) {
-  return (static_cast<uint32_t>(count) << 16) | (0xffffu - static_cast<uint32_t>(s));
-}
+// then lower slot); never 0, the value of an empty entry of a key list.  In 64
+// bits, or in 32 for count < 65536 and s < 65536.
+template <typename K>
+struct HeavyKey {
+  static constexpr int kBits = 4 * sizeof(K);  // of the slot, in the lower half
+  static constexpr K kLow = (static_cast<K>(1) << kBits) - 1;
+  static __device__ __forceinline__ K of(int count, int s) {
+    return (static_cast<K>(count) << kBits) | (kLow - static_cast<K>(s));
+  }
+  static __device__ __forceinline__ int slot(K key) { return static_cast<int>(kLow - (key & kLow)); }
+};
 
 // Rank of key among the kMaxHeavy entries of an LDS key list (empty entries
 // 0): the reads are independent, so all of them are in flight at once.
@@ -188,7 +190,7 @@ __device__ void scan_slots(int* hist, int P, int block_m, int* scan_lds,
     int h = hlpre >> 16;
     for (int i = 0; i < per; ++i) {
       const int s = s0 + i;
-      if (s < P && heavy_slot(hist[s], ctot)) heavy_keys[h++] = heavy_key(hist[s], s);
+      if (s < P && heavy_slot(hist[s], ctot)) heavy_keys[h++] = HeavyKey<uint64_t>::of(hist[s], s);
     }
   }
   // the scan's barriers also publish the keys (and, in the one before,
@@ -202,7 +204,7 @@ __device__ void scan_slots(int* hist, int P, int block_m, int* scan_lds,
         counts[s] = c;
         offsets[s] = cpre;
         tile_off[s] = tpre;
-        if (__builtin_expect(heavy_slot(c, ctot), 0)) active[heavy_rank(heavy_keys, heavy_key(c, s))] = s;
+        if (__builtin_expect(heavy_slot(c, ctot), 0)) active[heavy_rank(heavy_keys, HeavyKey<uint64_t>::of(c, s))] = s;
         else if (c > 0) active[lpre++] = s;
       }
       hist[s] = cpre;
@@ -309,32 +311,145 @@ __device__ __forceinline__ void permute_block(
 constexpr int kWavePermMaxSlotsPerLane = 16;
 constexpr int kWavePermMaxPairsPerLane = 4;
 
-// Per-slot outputs of one lane's slots s0 .. s0 + SPL - 1 (counts c, running
-// pair and tile prefixes cpre / tpre): counts, offsets, tile_off, the slot's
-// running base in lds, and the active entry of each slot with pairs at
-// positions lpos, lpos + 1, ...; with SKIP_HEAVY the heavy slots are left out
-// (the caller lists them).
-template <int SPL, bool SKIP_HEAVY>
-__device__ __forceinline__ void wave_slot_outputs(const int (&c)[SPL], int s0, int P, int block_m,
-                                                  int ctot, int cpre, int tpre, int lpos,
-                                                  int32_t* __restrict__ counts,
-                                                  int32_t* __restrict__ offsets,
-                                                  int32_t* __restrict__ tile_off,
-                                                  int32_t* __restrict__ active, int* lds) {
+// The slot scan of one wave over P <= 64 * SPL counts in LDS: lane `lane` owns
+// slots SPL lane .. SPL lane + SPL - 1.
+template <int SPL>
+struct SlotScan {
+  int c[SPL];  // counts
+  int cpre;    // pairs in the slots before this lane's
+  int ctot;    // pairs placed
+
+  // counts in lds -> this lane's prefix; lds then holds each slot's first
+  // position
+  __device__ __forceinline__ void begin(int* lds, int P) {
+    const int lane = threadIdx.x & 63;
+    const int s0 = lane * SPL;
+    int csum = 0;
 #pragma unroll
-  for (int i = 0; i < SPL; ++i) {
-    const int sl = s0 + i;
-    if (sl < P) {
-      counts[sl] = c[i];
-      offsets[sl] = cpre;
-      tile_off[sl] = tpre;
-      if (c[i] > 0 && !(SKIP_HEAVY && heavy_slot(c[i], ctot))) active[lpos++] = sl;
-      lds[sl] = cpre;  // running base of the slot
-      cpre += c[i];
-      tpre += (c[i] + block_m - 1) / block_m;
+    for (int i = 0; i < SPL; ++i) {
+      c[i] = (s0 + i < P) ? lds[s0 + i] : 0;
+      csum += c[i];
+    }
+    const int cinc = wave_inclusive_sum(csum);
+    cpre = cinc - csum;
+    ctot = read_lane_i32(cinc, 63);
+    wave_lds_sync();  // every lane has read its counts
+    int base = cpre;
+#pragma unroll
+    for (int i = 0; i < SPL; ++i) {
+      if (s0 + i < P) lds[s0 + i] = base;
+      base += c[i];
     }
   }
-}
+
+  // counts, offsets, tile_off, and the active entry of each slot with pairs
+  // at positions lpos, lpos + 1, ...; with SKIP_HEAVY the heavy slots are left
+  // out (the caller lists them).
+  template <bool SKIP_HEAVY>
+  __device__ __forceinline__ void slot_outputs(int P, int block_m, int tpre, int lpos,
+                                               int32_t* __restrict__ counts,
+                                               int32_t* __restrict__ offsets,
+                                               int32_t* __restrict__ tile_off,
+                                               int32_t* __restrict__ active) const {
+    const int s0 = (threadIdx.x & 63) * SPL;
+    int pre = cpre;
+#pragma unroll
+    for (int i = 0; i < SPL; ++i) {
+      const int sl = s0 + i;
+      if (sl < P) {
+        counts[sl] = c[i];
+        offsets[sl] = pre;
+        tile_off[sl] = tpre;
+        if (c[i] > 0 && !(SKIP_HEAVY && heavy_slot(c[i], ctot))) active[lpos++] = sl;
+        pre += c[i];
+        tpre += (c[i] + block_m - 1) / block_m;
+      }
+    }
+  }
+
+  // every output of the scan (N: an upper bound of the pairs; keys: kMaxHeavy
+  // entries of LDS for the heavy slots, uint32_t where N < 65536)
+  template <typename K>
+  __device__ __forceinline__ void publish(int N, int P, int block_m, int errs, K* keys,
+                                          int32_t* __restrict__ counts,
+                                          int32_t* __restrict__ offsets,
+                                          int32_t* __restrict__ active,
+                                          int32_t* __restrict__ tile_off,
+                                          int32_t* __restrict__ meta) const {
+    const int lane = threadIdx.x & 63;
+    const int s0 = lane * SPL;
+    int asum = 0, tsum = 0;
+#pragma unroll
+    for (int i = 0; i < SPL; ++i) {
+      asum += c[i] > 0;
+      tsum += (c[i] + block_m - 1) / block_m;
+    }
+    // launch order (heavy_slot): whether the wave holds a heavy slot (one
+    // ballot; the rare heavy case counts them again)
+    bool lane_heavy = false;
+#pragma unroll
+    for (int i = 0; i < SPL; ++i) lane_heavy |= heavy_slot(c[i], ctot);
+    const bool any_heavy = __builtin_amdgcn_ballot_w64(lane_heavy) != 0ull;
+    int apre, atot, tpre, ttot;
+    if constexpr (SPL == 1) {
+      // one slot per lane: the active prefix is a ballot count
+      const uint64_t am = __builtin_amdgcn_ballot_w64(asum > 0);
+      apre = static_cast<int>(__popcll(am & lanemask_lt(lane)));
+      atot = static_cast<int>(__popcll(am));
+    } else {
+      const int ainc = wave_inclusive_sum(asum);
+      apre = ainc - asum;
+      atot = read_lane_i32(ainc, 63);
+    }
+    if (SPL == 1 && N <= block_m) {
+      // no slot holds more than block_m pairs: one tile per active slot, so
+      // the tile prefix is the active prefix in slot order
+      tpre = apre;
+      ttot = atot;
+    } else {
+      const int tinc = wave_inclusive_sum(tsum);
+      tpre = tinc - tsum;
+      ttot = read_lane_i32(tinc, 63);
+    }
+    // uniform; marked unlikely so that the branch is laid out after the
+    // kernel's straight-line path
+    if (__builtin_expect(any_heavy, 0)) {
+      // heavy keys in slot order, empty entries 0; lane j < nh ranks key j
+      // against all of them and lists its slot.  Light slots follow the nh
+      // heavy ones: active slots before this lane's, less the heavy ones.
+      int hsum = 0;
+#pragma unroll
+      for (int i = 0; i < SPL; ++i) hsum += heavy_slot(c[i], ctot);
+      const int hinc = wave_inclusive_sum(hsum);
+      const int hpre = hinc - hsum;
+      const int nh = read_lane_i32(hinc, 63);
+      if (lane < kMaxHeavy && lane >= nh) keys[lane] = 0;
+      int h = hpre;
+#pragma unroll
+      for (int i = 0; i < SPL; ++i)
+        if (heavy_slot(c[i], ctot)) keys[h++] = HeavyKey<K>::of(c[i], s0 + i);
+      wave_lds_sync();
+      if (lane < nh) {
+        const K key = keys[lane];
+        active[heavy_rank(keys, key)] = HeavyKey<K>::slot(key);
+      }
+      slot_outputs<true>(P, block_m, tpre, apre + nh - hpre, counts, offsets, tile_off, active);
+    } else {
+      slot_outputs<false>(P, block_m, tpre, apre, counts, offsets, tile_off, active);
+    }
+    // active[a] = -1 past the active slots (see scan_slots)
+    for (int a = atot + lane; a < P; a += kWave) active[a] = -1;
+    if (lane == 0) {
+      offsets[P] = ctot;
+      tile_off[P] = ttot;
+      meta[LMOE_META_ACTIVE] = atot;
+      meta[LMOE_META_PAIRS] = ctot;
+      meta[LMOE_META_ERRORS] = errs;
+      meta[LMOE_META_TILES] = ttot;
+      publish_build(meta);
+    }
+  }
+};
 
 template <int SPL, int PPL>
 __device__ __forceinline__ void permute_wave(
@@ -372,91 +487,11 @@ __device__ __forceinline__ void permute_wave(
     }
   }
   wave_lds_sync();
-  // this lane's slots s0 .. s0+SPL-1: counts, then wave-wide prefixes
-  const int s0 = lane * SPL;
-  int c[SPL];
-  int csum = 0, asum = 0, tsum = 0;
-#pragma unroll
-  for (int i = 0; i < SPL; ++i) {
-    c[i] = (s0 + i < P) ? lds[s0 + i] : 0;
-    csum += c[i];
-    asum += c[i] > 0;
-    tsum += (c[i] + block_m - 1) / block_m;
-  }
-  const int cinc = wave_inclusive_sum(csum);
-  int cpre = cinc - csum;
-  const int ctot = read_lane_i32(cinc, 63);
-  // launch order (heavy_slot): whether the wave holds a heavy slot (one
-  // ballot; the rare heavy case counts them again)
-  bool lane_heavy = false;
-#pragma unroll
-  for (int i = 0; i < SPL; ++i) lane_heavy |= heavy_slot(c[i], ctot);
-  const bool any_heavy = __builtin_amdgcn_ballot_w64(lane_heavy) != 0ull;
-  int apre, atot, tpre, ttot;
-  if constexpr (SPL == 1) {
-    // one slot per lane: the active prefix is a ballot count
-    const uint64_t am = __builtin_amdgcn_ballot_w64(asum > 0);
-    apre = static_cast<int>(__popcll(am & lanemask_lt(lane)));
-    atot = static_cast<int>(__popcll(am));
-  } else {
-    const int ainc = wave_inclusive_sum(asum);
-    apre = ainc - asum;
-    atot = read_lane_i32(ainc, 63);
-  }
-  if (SPL == 1 && N <= block_m) {
-    // no slot holds more than block_m pairs: one tile per active slot, so
-    // the tile prefix is the active prefix in slot order
-    tpre = apre;
-    ttot = atot;
-  } else {
-    const int tinc = wave_inclusive_sum(tsum);
-    tpre = tinc - tsum;
-    ttot = read_lane_i32(tinc, 63);
-  }
-  // uniform; marked unlikely so that the branch is laid out after the
-  // kernel's straight-line path
-  if (__builtin_expect(any_heavy, 0)) {
-    // heavy keys in lds[64 SPL .. + kMaxHeavy) (slot order, empty entries
-    // 0); lane j < nh ranks key j against all of them and lists its slot.
-    // Light slots follow the nh heavy ones: active slots before this lane's,
-    // less the heavy ones.  (counts <= N <= 256 and slots < 1024 here:
-    // 32-bit keys)
-    int hsum = 0;
-#pragma unroll
-    for (int i = 0; i < SPL; ++i) hsum += heavy_slot(c[i], ctot);
-    const int hinc = wave_inclusive_sum(hsum);
-    const int hpre = hinc - hsum;
-    const int nh = read_lane_i32(hinc, 63);
-    uint32_t* keys = reinterpret_cast<uint32_t*>(lds + kWave * SPL);
-    if (lane < kMaxHeavy && lane >= nh) keys[lane] = 0;
-    int h = hpre;
-#pragma unroll
-    for (int i = 0; i < SPL; ++i)
-      if (heavy_slot(c[i], ctot)) keys[h++] = heavy_key16(c[i], s0 + i);
-    wave_lds_sync();
-    if (lane < nh) {
-      const uint32_t key = keys[lane];
-      active[heavy_rank(keys, key)] = static_cast<int>(0xffffu - (key & 0xffffu));
-    }
-    wave_lds_sync();  // every lane has read its counts and the keys before lds is reused
-    wave_slot_outputs<SPL, true>(c, s0, P, block_m, ctot, cpre, tpre, apre + nh - hpre, counts,
-                                 offsets, tile_off, active, lds);
-  } else {
-    wave_lds_sync();  // every lane has read its counts before lds is reused
-    wave_slot_outputs<SPL, false>(c, s0, P, block_m, ctot, cpre, tpre, apre, counts, offsets,
-                                  tile_off, active, lds);
-  }
-  // active[a] = -1 past the active slots (see scan_slots)
-  for (int a = atot + lane; a < P; a += kWave) active[a] = -1;
-  if (lane == 0) {
-    offsets[P] = ctot;
-    tile_off[P] = ttot;
-    meta[LMOE_META_ACTIVE] = atot;
-    meta[LMOE_META_PAIRS] = ctot;
-    meta[LMOE_META_ERRORS] = errs;
-    meta[LMOE_META_TILES] = ttot;
-    publish_build(meta);
-  }
+  SlotScan<SPL> scan;
+  scan.begin(lds, P);
+  // (counts <= N <= 256 here: 32-bit keys)
+  scan.publish(N, P, block_m, errs, reinterpret_cast<uint32_t*>(lds + kWave * SPL), counts,
+               offsets, active, tile_off, meta);
   // groups in flat order: read the slot's running base, then its first
   // pair of the group advances it past the group's pairs
 #pragma unroll
@@ -521,6 +556,115 @@ __device__ __forceinline__ void permute_wave_any(
   else if (spl == 8) LMOE_PW(8);
   else LMOE_PW(16);
 #undef LMOE_PW
+}
+
+// ---------------------------------------------------------------------------
+// The block permutations with a count table: each wave ranks its 64 pairs with
+// ballots and stores how many it has of each slot in a row of its own; the
+// rows' prefixes give every pair its position at once, where chunk_positions
+// lets one wave after the other advance the slots' running bases (a barrier and
+// an LDS round trip per wave), and one wave scans the slots without the block
+// scans' barriers: three or four barriers instead of up to 29.  Bound by that
+// chain's latency (launch, ids, slot table, scan).
+// ---------------------------------------------------------------------------
+// rows: [waves][64 spl] uint16; this wave's row is cleared and filled, the rank
+// of this lane's pair (slot s, < 0 for none) in its wave returned
+__device__ __forceinline__ int wave_row_counts(int s, int P, int spl, uint16_t* rows) {
+  const int lane = threadIdx.x & 63;
+  uint16_t* row = rows + static_cast<size_t>(threadIdx.x >> 6) * kWave * spl;
+  for (int i = lane; i < kWave / 2 * spl; i += kWave) reinterpret_cast<uint32_t*>(row)[i] = 0;
+  const int nbits = key_bits(P);
+  const bool placed = s >= 0;
+  const uint64_t m = match_key(placed ? s : (1 << nbits) - 1, nbits);
+  const int rank = __popcll(m & lanemask_lt(lane));
+  wave_lds_sync();
+  if (placed && rank == 0) row[s] = static_cast<uint16_t>(__popcll(m));
+  return rank;
+}
+
+// Each row's counts -> the counts of the rows before it (two slots per word:
+// no sum passes kChunk, so none carries into the upper half); TOTALS: totals[s]
+// = the slot's count over all rows
+template <bool TOTALS>
+__device__ __forceinline__ void row_prefixes(uint16_t* rows, int spl, int* totals) {
+  const int nw = blockDim.x >> 6;
+  const int words = kWave / 2 * spl;
+  uint32_t* r = reinterpret_cast<uint32_t*>(rows);
+  for (int i = threadIdx.x; i < words; i += blockDim.x) {
+    uint32_t v[kChunk / kWave];
+#pragma unroll
+    for (int w = 0; w < kChunk / kWave; ++w) v[w] = w < nw ? r[w * words + i] : 0u;
+    uint32_t run = 0;
+#pragma unroll
+    for (int w = 0; w < kChunk / kWave; ++w) {
+      if (w < nw) r[w * words + i] = run;
+      run += v[w];
+    }
+    if (TOTALS) {
+      totals[2 * i] = static_cast<int>(run & 0xffffu);
+      totals[2 * i + 1] = static_cast<int>(run >> 16);
+    }
+  }
+}
+
+// LDS ints of permute_block_table: totals, heavy keys, errors per wave, rows
+__host__ __device__ inline int table_perm_lds_ints(int P, int threads) {
+  const int pl = kWave * wave_perm_spl(P);
+  return pl + kMaxHeavy + kChunk / kWave + threads / kWave * pl / 2;
+}
+
+// Whole permutation of N <= blockDim.x pairs over P <= 512 slots by one block:
+// the outputs of permute_block.  lds: table_perm_lds_ints(P, blockDim.x) ints.
+template <int SPL>
+__device__ __forceinline__ void permute_block_table(
+    const int32_t* ids, int N, const int32_t* __restrict__ log2phy, int n_log2phy, int P,
+    int skip, int block_m, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
+    int32_t* __restrict__ sorted_pairs, int32_t* __restrict__ row_idx,
+    int32_t* __restrict__ active, int32_t* __restrict__ tile_off, int32_t* __restrict__ meta,
+    int* lds, RowKeep keep) {
+  uint32_t* keys = reinterpret_cast<uint32_t*>(lds + kWave * SPL);  // N <= kChunk: 32 bits
+  int* wave_errs = lds + kWave * SPL + kMaxHeavy;
+  uint16_t* rows = reinterpret_cast<uint16_t*>(wave_errs + kChunk / kWave);
+  const int p = threadIdx.x;
+  const int lane = p & 63;
+  const int wave = p >> 6;
+  const int s = p < N ? map_pair(ids, p, log2phy, n_log2phy, P, skip) : -1;
+  const int errs = __popcll(__ballot(s == -2));
+  if (lane == 0) wave_errs[wave] = errs;
+  const int rank = wave_row_counts(s, P, SPL, rows);
+  __syncthreads();
+  row_prefixes<true>(rows, SPL, lds);
+  __syncthreads();
+  SlotScan<SPL> scan;
+  if (wave == 0) scan.begin(lds, P);
+  __syncthreads();
+  if (p < N) {
+    const int pos = s >= 0 ? lds[s] + rows[wave * kWave * SPL + s] + rank : -1;
+    if ((pos >= 0 || skip != kSkipKeepRows) && !kept_row(keep, ids, p)) row_idx[p] = pos;
+    if (pos >= 0) sorted_pairs[pos] = p;
+  }
+  if (wave == 0) {
+    const int e = wave_inclusive_sum(lane < static_cast<int>(blockDim.x >> 6) ? wave_errs[lane] : 0);
+    scan.publish(N, P, block_m, read_lane_i32(e, 63), keys, counts, offsets, active, tile_off,
+                 meta);
+  }
+}
+
+__device__ __forceinline__ void permute_block_table_any(
+    const int32_t* ids, int N, const int32_t* __restrict__ log2phy, int n_log2phy, int P,
+    int skip, int block_m, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
+    int32_t* __restrict__ sorted_pairs, int32_t* __restrict__ row_idx,
+    int32_t* __restrict__ active, int32_t* __restrict__ tile_off, int32_t* __restrict__ meta,
+    int* lds, RowKeep keep = {}) {
+  const int spl = wave_perm_spl(P);
+#define LMOE_PBT(S)                                                                             \
+  permute_block_table<S>(ids, N, log2phy, n_log2phy, P, skip, block_m, counts, offsets,         \
+                         sorted_pairs, row_idx, active, tile_off, meta, lds, keep)
+  if (spl <= 1) LMOE_PBT(1);
+  else if (spl == 2) LMOE_PBT(2);
+  else if (spl == 4) LMOE_PBT(4);
+  else LMOE_PBT(8);
+#undef LMOE_PBT
 }
 
 }  // namespace lmoe

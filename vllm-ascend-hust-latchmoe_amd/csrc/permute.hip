@@ -3,18 +3,25 @@
 
 namespace lmoe {
 
-// Whole permutation in one block (n_pairs <= kChunk).
+// Whole permutation in one block (n_pairs <= kChunk).  TABLE: the form with a
+// count table.
+template <bool TABLE>
 __global__ __launch_bounds__(1024) void permute_small_kernel(
     const int32_t* __restrict__ ids, int N, const int32_t* __restrict__ log2phy,
     int n_log2phy, int P, int skip, int block_m, int32_t* __restrict__ counts,
     int32_t* __restrict__ offsets, int32_t* __restrict__ sorted_pairs,
     int32_t* __restrict__ row_idx, int32_t* __restrict__ active,
     int32_t* __restrict__ tile_off, int32_t* __restrict__ meta) {
-  extern __shared__ int hist[];  // [P]
-  __shared__ int scan_lds[33];
-  __shared__ int err_lds;
-  permute_block(ids, N, log2phy, n_log2phy, P, skip, block_m, counts, offsets, sorted_pairs,
-                row_idx, active, tile_off, meta, hist, scan_lds, &err_lds);
+  extern __shared__ int hist[];  // [P], TABLE: [table_perm_lds_ints(P, threads)]
+  if constexpr (TABLE) {
+    permute_block_table_any(ids, N, log2phy, n_log2phy, P, skip, block_m, counts, offsets,
+                            sorted_pairs, row_idx, active, tile_off, meta, hist);
+  } else {
+    __shared__ int scan_lds[33];
+    __shared__ int err_lds;
+    permute_block(ids, N, log2phy, n_log2phy, P, skip, block_m, counts, offsets, sorted_pairs,
+                  row_idx, active, tile_off, meta, hist, scan_lds, &err_lds);
+  }
 }
 
 // Whole permutation by one wave (n_pairs <= 64 * PPL, n_slots <= 1024).
@@ -57,17 +64,25 @@ __device__ __forceinline__ RowKeep keep_of(bool second, const PermBuild& b) {
   return k;
 }
 
+template <bool TABLE>
 __global__ __launch_bounds__(1024) void permute_small_two_kernel(
     const int32_t* __restrict__ ids, int N, int block_m, PermBuild a, PermBuild b,
     int32_t* __restrict__ row_idx) {
-  extern __shared__ int hist[];  // [max(P_a, P_b)]
-  __shared__ int scan_lds[33];
-  __shared__ int err_lds;
+  extern __shared__ int hist[];  // the larger of the two tables' (permute_small_kernel)
   const bool second = blockIdx.x != 0;
   const PermBuild o = second ? b : a;
-  permute_block(ids, N, o.log2phy, o.n_log2phy, o.P, second ? kSkipKeepRows : 1, block_m,
-                o.counts, o.offsets, o.sorted_pairs, row_idx, o.active, o.tile_off, o.meta, hist,
-                scan_lds, &err_lds, keep_of(second, b));
+  const int skip = second ? kSkipKeepRows : 1;
+  if constexpr (TABLE) {
+    permute_block_table_any(ids, N, o.log2phy, o.n_log2phy, o.P, skip, block_m, o.counts,
+                            o.offsets, o.sorted_pairs, row_idx, o.active, o.tile_off, o.meta,
+                            hist, keep_of(second, b));
+  } else {
+    __shared__ int scan_lds[33];
+    __shared__ int err_lds;
+    permute_block(ids, N, o.log2phy, o.n_log2phy, o.P, skip, block_m, o.counts, o.offsets,
+                  o.sorted_pairs, row_idx, o.active, o.tile_off, o.meta, hist, scan_lds,
+                  &err_lds, keep_of(second, b));
+  }
 }
 
 template <int PPL>
@@ -158,6 +173,86 @@ __global__ __launch_bounds__(1024) void permute_scan_scatter_kernel(
   }
 }
 
+// Step 2 with a count table (slots within wave_perm_spl): the same outputs.
+// All threads sum the chunks' counts (blockDim.x / (64 SPL) threads per slot,
+// each a share of the chunks), and the chunk's pairs are placed as in
+// permute_block_table.  LDS: scatter_table_lds_ints(P).
+template <int SPL>
+__device__ __forceinline__ void scan_scatter_table(
+    int N, int P, int nchunks, int skip, int block_m, const int32_t* __restrict__ slot_of,
+    const int32_t* __restrict__ chunk_cnt, const int32_t* __restrict__ chunk_err,
+    int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ active,
+    int32_t* __restrict__ tile_off, int32_t* __restrict__ meta,
+    int32_t* __restrict__ sorted_pairs, int32_t* __restrict__ row_idx, int* lds) {
+  constexpr int PL = kWave * SPL;
+  constexpr int PARTS = kChunk / PL;  // threads per slot
+  int* before = lds + PL;  // the counts of the chunks before this one
+  uint64_t* keys = reinterpret_cast<uint64_t*>(lds + 2 * PL);
+  uint16_t* rows = reinterpret_cast<uint16_t*>(lds + 2 * PL + 2 * kMaxHeavy);
+  const int c0 = blockIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int p = c0 * kChunk + threadIdx.x;
+  const int sp = p < N ? slot_of[p] : -1;
+  const int s = threadIdx.x & (PL - 1);
+  int tot = 0, pre = 0;
+  if (s < P) {
+#pragma unroll 8
+    for (int c = threadIdx.x / PL; c < nchunks; c += PARTS) {
+      const int v = chunk_cnt[static_cast<size_t>(c) * P + s];
+      tot += v;
+      pre += c < c0 ? v : 0;
+    }
+  }
+  if (PARTS > 1) {
+    if (threadIdx.x < PL) {
+      lds[s] = 0;
+      before[s] = 0;
+    }
+    __syncthreads();
+    if (tot != 0) atomicAdd(&lds[s], tot);
+    if (pre != 0) atomicAdd(&before[s], pre);
+  } else {
+    lds[s] = tot;
+    before[s] = pre;
+  }
+  const int rank = wave_row_counts(sp, P, SPL, rows);
+  __syncthreads();
+  SlotScan<SPL> scan;
+  if (wave == 0) scan.begin(lds, P);
+  row_prefixes<false>(rows, SPL, nullptr);
+  __syncthreads();
+  if (p < N) {
+    const int pos = sp >= 0 ? lds[sp] + before[sp] + rows[wave * PL + sp] + rank : -1;
+    if (pos >= 0 || skip != kSkipKeepRows) row_idx[p] = pos;
+    if (pos >= 0) sorted_pairs[pos] = p;
+  }
+  if (c0 == 0 && wave == 0) {
+    int e = 0;
+    for (int c = lane; c < nchunks; c += kWave) e += chunk_err[c];
+    e = wave_inclusive_sum(e);
+    scan.publish(N, P, block_m, read_lane_i32(e, 63), keys, counts, offsets, active, tile_off,
+                 meta);
+  }
+}
+
+static int scatter_table_lds_ints(int P) {
+  const int pl = kWave * wave_perm_spl(P);
+  return 2 * pl + 2 * kMaxHeavy + kChunk / kWave * pl / 2;
+}
+
+template <int SPL>
+__global__ __launch_bounds__(1024) void permute_scatter_table_kernel(
+    int N, int P, int nchunks, int skip, int block_m, const int32_t* __restrict__ slot_of,
+    const int32_t* __restrict__ chunk_cnt, const int32_t* __restrict__ chunk_err,
+    int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ active,
+    int32_t* __restrict__ tile_off, int32_t* __restrict__ meta,
+    int32_t* __restrict__ sorted_pairs, int32_t* __restrict__ row_idx) {
+  extern __shared__ __attribute__((aligned(8))) int lds[];
+  scan_scatter_table<SPL>(N, P, nchunks, skip, block_m, slot_of, chunk_cnt, chunk_err, counts,
+                          offsets, active, tile_off, meta, sorted_pairs, row_idx, lds);
+}
+
 // expanded_x rows
 __global__ __launch_bounds__(256) void gather_rows_kernel(
     const uint16_t* __restrict__ x, int H, int k,
@@ -176,6 +271,18 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(
 using namespace lmoe;
 
 static size_t align_up(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
+
+// Where the forms with a count table (permute.h) are the faster ones; their one
+// wave scans 64 slots per step, the other forms' block all of them.  Before ->
+// after, us per call in a graph:
+//   one block, 888 pairs: 128 slots 7.8 -> 6.0, 512 slots 8.1 -> 7.2, 768
+//     slots 8.2 -> 8.6; 257 pairs: 128 slots 6.0 -> 5.7, 320 slots 6.3 -> 6.7
+//   two tables of 112 and 16 slots, 888 pairs: 7.9 -> 5.8
+//   several blocks, 32768 pairs: 128 slots 13.4 -> 9.4, 1024 slots 14.6 -> 13.1
+static bool block_table_fits(int n_pairs, int n_slots) {
+  return n_slots <= 256 || (n_slots <= 512 && n_pairs > 512);
+}
+static bool scatter_table_fits(int n_slots) { return wave_perm_spl(n_slots) > 0; }
 
 extern "C" size_t lmoe_permute_workspace_bytes(int n_pairs, int n_slots) {
   if (n_pairs <= kChunk || n_slots <= 0) return 0;
@@ -222,10 +329,17 @@ extern "C" int lmoe_permute(const int32_t* ids, int n_pairs,
     int threads = n_pairs > n_slots / 16 ? n_pairs : n_slots / 16;
     threads = ((threads + 63) / 64) * 64;
     threads = threads < 64 ? 64 : (threads > kChunk ? kChunk : threads);
-    hipLaunchKernelGGL(permute_small_kernel, dim3(1), dim3(threads), lds, stream,
-                       ids, n_pairs, log2phy, n_log2phy, n_slots, skip, block_m,
-                       counts, offsets, sorted_pairs, row_idx, active, tile_off,
-                       meta);
+    if (block_table_fits(n_pairs, n_slots)) {
+      threads = (n_pairs + 63) / 64 * 64;  // (fewer than 257 pairs are one wave's)
+      const size_t tlds = sizeof(int) * static_cast<size_t>(table_perm_lds_ints(n_slots, threads));
+      hipLaunchKernelGGL(permute_small_kernel<true>, dim3(1), dim3(threads), tlds, stream, ids,
+                         n_pairs, log2phy, n_log2phy, n_slots, skip, block_m, counts, offsets,
+                         sorted_pairs, row_idx, active, tile_off, meta);
+    } else {
+      hipLaunchKernelGGL(permute_small_kernel<false>, dim3(1), dim3(threads), lds, stream, ids,
+                         n_pairs, log2phy, n_log2phy, n_slots, skip, block_m, counts, offsets,
+                         sorted_pairs, row_idx, active, tile_off, meta);
+    }
     LMOE_RETURN_LAUNCH();
   }
   if (workspace == nullptr ||
@@ -241,9 +355,23 @@ extern "C" int lmoe_permute(const int32_t* ids, int n_pairs,
   hipLaunchKernelGGL(permute_hist_kernel, dim3(nchunks), dim3(kChunk), lds,
                      stream, ids, n_pairs, log2phy, n_log2phy, n_slots, skip,
                      slot_of, chunk_cnt, chunk_err);
-  hipLaunchKernelGGL(permute_scan_scatter_kernel, dim3(nchunks), dim3(kChunk), 2 * lds, stream,
-                     n_pairs, n_slots, nchunks, skip, block_m, slot_of, chunk_cnt, chunk_err,
-                     counts, offsets, active, tile_off, meta, sorted_pairs, row_idx);
+#define LMOE_PSC(KERNEL, LDS)                                                                  \
+  hipLaunchKernelGGL(KERNEL, dim3(nchunks), dim3(kChunk), LDS, stream, n_pairs, n_slots, nchunks, \
+                     skip, block_m, slot_of, chunk_cnt, chunk_err, counts, offsets, active,      \
+                     tile_off, meta, sorted_pairs, row_idx)
+  if (scatter_table_fits(n_slots)) {
+    const size_t tlds = sizeof(int) * static_cast<size_t>(scatter_table_lds_ints(n_slots));
+    switch (wave_perm_spl(n_slots)) {
+      case 1: LMOE_PSC(permute_scatter_table_kernel<1>, tlds); break;
+      case 2: LMOE_PSC(permute_scatter_table_kernel<2>, tlds); break;
+      case 4: LMOE_PSC(permute_scatter_table_kernel<4>, tlds); break;
+      case 8: LMOE_PSC(permute_scatter_table_kernel<8>, tlds); break;
+      default: LMOE_PSC(permute_scatter_table_kernel<16>, tlds); break;
+    }
+  } else {
+    LMOE_PSC(permute_scan_scatter_kernel, 2 * lds);
+  }
+#undef LMOE_PSC
   LMOE_RETURN_LAUNCH();
 }
 
@@ -291,9 +419,16 @@ extern "C" int lmoe_permute_two_tables(
   int threads = n_pairs > P / 16 ? n_pairs : P / 16;
   threads = ((threads + 63) / 64) * 64;
   threads = threads < 64 ? 64 : (threads > kChunk ? kChunk : threads);
-  hipLaunchKernelGGL(permute_small_two_kernel, dim3(2), dim3(threads),
-                     sizeof(int) * static_cast<size_t>(P), stream, ids, n_pairs, block_m, a, b,
-                     row_idx);
+  if (block_table_fits(n_pairs, P)) {
+    threads = (n_pairs + 63) / 64 * 64;
+    const size_t tlds = sizeof(int) * static_cast<size_t>(table_perm_lds_ints(P, threads));
+    hipLaunchKernelGGL(permute_small_two_kernel<true>, dim3(2), dim3(threads), tlds, stream, ids,
+                       n_pairs, block_m, a, b, row_idx);
+  } else {
+    hipLaunchKernelGGL(permute_small_two_kernel<false>, dim3(2), dim3(threads),
+                       sizeof(int) * static_cast<size_t>(P), stream, ids, n_pairs, block_m, a, b,
+                       row_idx);
+  }
   LMOE_RETURN_LAUNCH();
 }
 
