@@ -36,7 +36,7 @@
 // Measured (Qwen3 shapes, 128 slots, gate-up + down): 64 tokens 182 us
 // (6.5 TB/s; GEMV 212, 320-row tiles 244), 300 tokens 207 us (247), 1024
 // tokens 245 us (269); DeepSeek-V3 expert shape, 700 tokens 3.56 ms (4.01),
-// 2048 tokens (72 per slot) 4.34 ms (4.59): there the token rows' loads and the
+// 2048 tokens (72 per slot) 4.26 ms (4.59): there the token rows' loads and the
 // output rows' stores take the time past the weight stream's 3.4 ms, not the
 // MFMAs or LDS (a copy without most of the MFMAs: 1% less).
 #pragma once
@@ -273,9 +273,9 @@ __device__ __forceinline__ int stream_tile_slot(const int32_t* tile_off, int P, 
 // then those of g2, whose act rows follow the pairs g places (an overflow
 // slot's rows stay inside the n_pairs rows of the act buffer).  Registers:
 // RT 1 leaves 4 waves per SIMD, RT 2 three, with the partial sums three and two
-// (two or three waves take the same time).
+// (two or three waves take the same time), RT 4 two.
 template <int MODE, int RT, bool SPLIT, bool TWO>
-__global__ __launch_bounds__(kStreamWaves * 64, RT == 2 && SPLIT ? 2 : RT == 1 && !SPLIT ? 4 : 3) void stream_gemm_kernel(
+__global__ __launch_bounds__(kStreamWaves * 64, RT == 4 || (RT == 2 && SPLIT) ? 2 : RT == 1 && !SPLIT ? 4 : 3) void stream_gemm_kernel(
     StreamArgs g, StreamArgs g2, int n_pairs) {
   __shared__ __attribute__((aligned(1024))) char
       smem[kStreamWaves * RT * 2048 + 2 * (kStreamBM / 16) * 2048];

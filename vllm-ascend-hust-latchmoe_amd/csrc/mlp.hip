@@ -925,6 +925,7 @@ static bool part_offsets_fit(const GemmArgs& g, int n_pairs) {
 // even out the last round: 128 slots of the Qwen3 shape 182 us wide against
 // 190 narrow, 64 slots at 40 tokens 123 against 113 (gate-up + down).
 constexpr long long kStreamWideBlocks = 1500;
+constexpr int kStreamWiderRows = 40;
 
 template <int MODE, bool SPLIT, bool TWO>
 static int launch_stream(const StreamArgs& a, const StreamArgs& b, int n_pairs, int max_active,
@@ -934,6 +935,23 @@ static int launch_stream(const StreamArgs& a, const StreamArgs& b, int n_pairs, 
   if (tiles > 65535) return LMOE_ERR_SHAPE;
   constexpr int wide_cols = kStreamWaves * (MODE == kGateUp ? 16 : 32);
   const int wide = (a.N + wide_cols - 1) / wide_cols;
+  if constexpr (MODE == kGateUp && !SPLIT && !TWO) {
+    // many rows per slot: twice the weight rows per block, so that a stage
+    // loads half the token rows per weight byte, while that still makes two
+    // blocks per CU.  Gate-up, before -> after (us): 257 slots of 72 rows, H
+    // 7168, I 2048: 2788 -> 2665; 64 of 62, H 4096, I 1024: 279 -> 246; 60 of
+    // 47, H 2048, I 1408: 165 -> 156; 128 of 64, H 2048, I 768: the same.  With
+    // fewer rows it is slower (128 of 19: 145 -> 157; 257 of 10: 2294 -> 2345),
+    // and the down GEMM (more output rows to store) gains nothing.
+    const int wider = (a.N + 2 * wide_cols - 1) / (2 * wide_cols);
+    if (n_pairs >= kStreamWiderRows * static_cast<long long>(a.P) &&
+        static_cast<long long>(wider) * max_active >= 512) {
+      hipLaunchKernelGGL((stream_gemm_kernel<MODE, 4, SPLIT, TWO>),
+                         dim3(wider, static_cast<unsigned>(tiles)), dim3(kStreamWaves * 64), 0,
+                         stream, a, b, n_pairs);
+      return LMOE_OK;
+    }
+  }
   if (static_cast<long long>(wide) * max_active >= kStreamWideBlocks)
     hipLaunchKernelGGL((stream_gemm_kernel<MODE, 2, SPLIT, TWO>),
                        dim3(wide, static_cast<unsigned>(tiles)), dim3(kStreamWaves * 64), 0, stream,
