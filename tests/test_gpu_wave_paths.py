@@ -1,0 +1,36 @@
+"""Prefill past the bank with few experts per wave: 33 tokens and more of up to
+1024 pairs take the streaming path with its one row-tile height, however many
+pairs a wave's slots hold.  Host- and device-planned waves give the full
+layer's bits (every path computes a pair's row alone), so no tolerance."""
+
+import pytest
+import torch
+
+from oracle.bf16 import normal_bf16
+from tests._util import to_dev_bf16
+from tests.test_gpu_device_waves import _layer
+
+pytestmark = pytest.mark.gpu
+
+
+# pairs per slot past STREAM_MAX_PAIRS_PER_SLOT: of the whole layer over a
+# host-planned wave's experts, and of one device-planned wave over the bank;
+# the GEMV, streaming and MFMA paths' first and last token counts
+@pytest.mark.parametrize("E,slots,T", [(64, 8, 100), (8, 2, 101), (8, 2, 32), (8, 2, 33), (8, 2, 128), (8, 2, 129)])
+def test_waves_of_few_experts_equal_the_full_layer(E, slots, T):
+    from vllm_moe_offload_amd import fused_moe
+
+    H = 1024
+    print(f"case waves E={E} slots={slots} T={T}", flush=True)
+    layer, rt, rng = _layer({}, E=E, slots=slots)
+    dx = to_dev_bf16(normal_bf16(rng, (T, H), 1.0))
+    w, ids, _ = fused_moe.route(dx, layer.gate_weight, layer.router_spec)
+    kw = dict(layer_id=layer.layer_id, hidden=dx, topk_weights=w, topk_ids=ids, num_logical_experts=E)
+    full = fused_moe.run_full_layer(rt, **kw).clone()
+    dev = fused_moe.run_device_waves(rt, **kw).clone()
+    host, report = fused_moe.run_wave_prefill(rt, **kw)
+    host = host.clone()
+    torch.cuda.synchronize()
+    assert len(report.waves) == E // slots
+    assert torch.equal(dev.view(torch.int16), full.view(torch.int16))
+    assert torch.equal(host.view(torch.int16), full.view(torch.int16))

@@ -172,16 +172,22 @@ def _overflow_perm(hidden, k: int, overflow: PreparedSlotWeights, ws: MoEWorkspa
     return ws.overflow_perm(hidden.shape[0] * k, int(overflow.physical_expert_count), hidden.device)
 
 
-def _block_m(hidden, k: int, w13_slots, path: int) -> int:
-    """The row-tile height to build a pass's permutation with (the GEMVs read
-    no tile table)."""
+def _pass_block_m(n_experts: int, H: int, I: int, device, n_pairs: int, path: int) -> int:
+    """The row-tile height to build the permutation of a pass over n_experts
+    slots with: the path's own (the GEMVs read no tile table, path STREAM has
+    one height), else the MFMA kernel's for n_pairs pairs."""
     if path == native.LMOE_PATH_GEMV:
         return native.MFMA_BLOCK_M
     if path == native.LMOE_PATH_STREAM:
         return native.STREAM_BLOCK_M
+    return native.prefill_block_m(n_experts, H, I, device, n_pairs=n_pairs)
+
+
+def _block_m(hidden, k: int, w13_slots, path: int) -> int:
+    """_pass_block_m of a pass over a whole bank."""
     T, H = hidden.shape
     P, I = int(w13_slots.shape[0]), int(w13_slots.shape[1]) // 2
-    return native.prefill_block_m(P, H, I, hidden.device, n_pairs=T * k)
+    return _pass_block_m(P, H, I, hidden.device, T * k, path)
 
 
 def _overflow_permute(hidden, topk_ids, k: int, overflow: PreparedSlotWeights, ws: MoEWorkspace, *,
@@ -656,6 +662,7 @@ def run_wave_prefill(
     profiling = bool(runtime.profile_path)
     wave_profiles: dict[int, dict] = {}
     ws = get_workspace(T, k, P, H, I, hidden.device, tag="waves")
+    mlp_path = _pass_path(T, k, H, I, path)
     report = WaveRunReport(plan.waves, sched.compute_order)
     staged: dict[int, tuple] = {}
     total_logical = runtime.total_logical_expert_count_for_layer(layer_id=layer_id, fallback=num_logical_experts)
@@ -706,10 +713,10 @@ def run_wave_prefill(
             try:
                 native.permute(topk_ids, ws.perm, log2phy=prepared.log2phy, skip_unmapped=True, keep_rows=not first,
                                table_len=total_logical if first else routed,
-                               block_m=native.prefill_block_m(len(plan.waves[w]), H, I, hidden.device, n_pairs=T * k))
+                               block_m=_pass_block_m(len(plan.waves[w]), H, I, hidden.device, T * k, mlp_path))
                 first = False
                 native.grouped_mlp(hidden, k, prepared.w1, prepared.w2, ws.perm, ws.act[: T * k], ws.y[: T * k],
-                                   path=_pass_path(T, k, H, I, path))
+                                   path=mlp_path)
             finally:
                 runtime.end_slot_compute(handle)
             if buf is not None:
@@ -881,7 +888,8 @@ def run_device_waves(
             if isinstance(ev, torch.cuda.Event):
                 tx.wait_event(ev)
     released: list = [None] * len(stages)
-    bm = native.prefill_block_m(P, H, I, dev, n_pairs=-(-(T * k) // n_waves))
+    mlp_path = _pass_path(T, k, H, I, path)
+    bm = _pass_block_m(P, H, I, dev, -(-(T * k) // n_waves), mlp_path)
     for w in range(n_waves):
         b = w % len(stages)
         stage, table = stages[b], tables[b]
@@ -896,7 +904,7 @@ def run_device_waves(
         compute.wait_event(ready)
         native.permute(topk_ids, ws.perm, log2phy=table, skip_unmapped=True, keep_rows=w > 0, block_m=bm)
         native.grouped_mlp(hidden, k, stage.w13_slots, stage.w2_slots, ws.perm, ws.act[: T * k], ws.y[: T * k],
-                           path=_pass_path(T, k, H, I, path))
+                           path=mlp_path)
         done = torch.cuda.Event()
         done.record(compute)
         released[b] = done
