@@ -631,7 +631,11 @@ DECODE_GEMV_MAX_TOKENS = 32
 # per slot) 245 / 269, 1300 (81) 272 / 274, 1600 (100) 400 / 285, with half the
 # rank bias 800 tokens 269 / 317, 1300 330 / 341; Qwen1.5-MoE, the same bias,
 # 400 tokens (27 pairs) 210 / 246, 800 (53) 267 / 258; DeepSeek-V3 shape 1024
-# tokens (36 pairs) 3734 / 4127, 2048 (72) 4341 / 4590.
+# tokens (36 pairs) 3734 / 4127, 2048 (72) 4341 / 4590.  With the whole rank
+# bias, hot slots of several tiles sharing their weights through the L2: Qwen3
+# 600 tokens 247 / 289, 1200 318 / 363; Qwen1.5-MoE 800 258 / 286, 1100 (73
+# pairs) 294 / 299; DeepSeek-V3 1100 3851 / 4116, 2048 4579 / 4749.  Equal
+# near the line without a bias (Qwen1.5-MoE, 1100 tokens 243 / 240).
 STREAM_MAX_PAIRS_PER_SLOT = 75
 
 
