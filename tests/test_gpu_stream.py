@@ -60,6 +60,7 @@ def _run(native, d_x, k, w13, w2, d_ids, l2p, bm, n_slots, skip=False, path=None
     (64, 1088, [16, 17, 33, 48, 64, 65, 96, 97, 0, 150] * 6),  # 58 rows per slot, 540 blocks of 128 columns
     (1024, 1024, [97, 300, 5, 193, 96]),  # slots of several row tiles, column blocks a multiple of 8
     (192, 320, [1, 17, 66] * 101),     # 303 slots of 5 column blocks: the wide form
+    (2112, 448, [5, 40, 97]),          # 33 K steps: the first past two phases in gate-up
 ])
 def test_stream_tiles_equal_128_row_tiles_and_oracle(H, I, counts):
     native = _native()

@@ -51,16 +51,25 @@ struct GemmArgs {
   int out_f32;            // dense only
 };
 
-// The K step (of KT 64-column steps) that an output column starts from: 128
-// act columns (gate-up) or 256 output columns (down) share one of four
-// phases, the K loop wraps around.  Rows of 4096 bytes walked in step by all
-// workgroups keep to a few memory channels at a time; with the phases the
-// Qwen3-shaped gate-up of few tokens per slot streams at 6.5 instead of 5.9
-// TB/s.  Every grouped kernel takes a column's steps in this order, so they
-// agree bit for bit.
+// The K step (of KT 64-column steps) that an output column starts from; the K
+// loop wraps around.  Rows of 4096 bytes walked in step by all workgroups keep
+// to a few memory channels at a time.  Blocks of 256 output columns (down) and,
+// for K > 2048, of 128 act columns (gate-up) take four phases of KT / 4 in turn.
+// Gate-up with K <= 2048 takes two, 0 and KT / 2, its blocks going 0 1 1 0 0 1
+// 1 ...: two of three neighbours, the 320-row kernel's units that read the same
+// activation rows through one L2, start together, and half of any few blocks
+// start late.  Every grouped kernel takes a column's steps in this order, so
+// they agree bit for bit.  Gate-up, us (one phase / four in turn / the above),
+// rows per slot evenly spread:
+//   H 2048, I 768, 128 slots   4 rows 133 / 119 / 118, 19  141 / 124 / 122,
+//       69  179 / 146 / 144 (96-row tiles); 188  211 / 217 / 215,
+//       256  245.9 / 249.9 / 242.5 (320-row tiles)
+//   H 2048, I 1408, 60 slots   73 rows 162 / 134 / 134; 273  237 / 237 / 236
+//   H 4096, I 1024, 64 slots   4 rows 194 / 159 / 159 (two phases 177)
 template <int MODE>
 __device__ __forceinline__ int k_phase(int col, int KT) {
   if (MODE == kDense) return 0;
+  if (MODE == kGateUp && KT <= 32) return ((((col >> 7) + 1) >> 1) & 1) * (KT >> 1);
   return ((col >> (MODE == kGateUp ? 7 : 8)) & 3) * (KT >> 2);
 }
 

@@ -19,7 +19,7 @@
 // Gate-up: a tile is 8 gate rows and the 8 matching up rows, so the halves of
 // a wave hold gate and up of the same 8 act columns.
 //
-// Each output column starts its K loop at one of four phases (k_phase): waves
+// Each output column starts its K loop at a phase of its own (k_phase): waves
 // that walk rows of 4096 bytes in step all read the same 1/16 of the memory
 // channels at a time.  A plain read of 805 MB in this access pattern took
 // 140 us in step and 116 us with four phases (6.95 TB/s).
