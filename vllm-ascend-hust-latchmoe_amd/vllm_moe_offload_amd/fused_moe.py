@@ -160,11 +160,12 @@ def fused_experts(
                              path=path, workspace=workspace)[0]
 
 
-def _pass_path(T: int, k: int, H: int, I: int, path: int) -> int:
-    """The MLP path of one pass of a multi-pass layer, by the rule the
-    single-pass layer uses (fused_experts), so a split layer gives the
-    unsplit layer's bits."""
-    return native.layer_path(T, k, H, I) if path == native.LMOE_PATH_AUTO else path
+def _layer_path(hidden, k: int, *w13) -> int:
+    """native.layer_path of a layer over the gate-up banks w13 (a pass's own
+    and, where there are several passes, all of them): one path for every
+    pass, so a split layer gives the unsplit layer's bits."""
+    T, H = hidden.shape
+    return native.layer_path(T, k, H, int(w13[0].shape[1]) // 2, aligned=native.aligned16(hidden, *w13))
 
 
 def _overflow_perm(hidden, k: int, overflow: PreparedSlotWeights, ws: MoEWorkspace) -> native.Permutation:
@@ -250,7 +251,7 @@ def _fused_experts_ws(hidden, topk_weights, topk_ids, w13_slots, w2_slots, log2p
     ws = workspace or get_workspace(T, k, P, H, I, hidden.device)
     dst = out if out is not None else ws.out[:T]
     if path == native.LMOE_PATH_AUTO:
-        path = native.layer_path(T, k, H, I)
+        path = _layer_path(hidden, k, w13_slots, *([overflow.w1] if overflow is not None else []))
     # the decode body; past its pair count path GEMV runs the two GEMVs apart
     decode = path == native.LMOE_PATH_GEMV and T * k <= native.FUSED_DECODE_MAX_PAIRS
     bm = _block_m(hidden, k, w13_slots, path)
@@ -348,8 +349,7 @@ def decode_layer(
         renormalize=bool(spec.renormalize), routed_scaling_factor=float(spec.routed_scaling_factor),
         n_shared=int(spec.n_shared), w_bf16=w_out, ids=ids_out, skip_unmapped=overflow is not None,
     )
-    I = int(w13_slots.shape[1]) // 2
-    path = native.layer_path(T, kw, int(hidden.shape[1]), I)
+    path = _layer_path(hidden, kw, w13_slots, *([overflow.w1] if overflow is not None else []))
     bm = _block_m(hidden, kw, w13_slots, path)
     merged = overflow is not None and log2phy is not None and _merged_passes(hidden, kw, w13_slots, overflow, path)
     perm_b = None
@@ -662,7 +662,7 @@ def run_wave_prefill(
     profiling = bool(runtime.profile_path)
     wave_profiles: dict[int, dict] = {}
     ws = get_workspace(T, k, P, H, I, hidden.device, tag="waves")
-    mlp_path = _pass_path(T, k, H, I, path)
+    mlp_path = _layer_path(hidden, k, bank.w13_slots) if path == native.LMOE_PATH_AUTO else path
     report = WaveRunReport(plan.waves, sched.compute_order)
     staged: dict[int, tuple] = {}
     total_logical = runtime.total_logical_expert_count_for_layer(layer_id=layer_id, fallback=num_logical_experts)
@@ -888,7 +888,7 @@ def run_device_waves(
             if isinstance(ev, torch.cuda.Event):
                 tx.wait_event(ev)
     released: list = [None] * len(stages)
-    mlp_path = _pass_path(T, k, H, I, path)
+    mlp_path = _layer_path(hidden, k, bank.w13_slots) if path == native.LMOE_PATH_AUTO else path
     bm = _pass_block_m(P, H, I, dev, -(-(T * k) // n_waves), mlp_path)
     for w in range(n_waves):
         b = w % len(stages)

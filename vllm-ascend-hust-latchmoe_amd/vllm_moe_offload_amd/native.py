@@ -639,17 +639,23 @@ DECODE_GEMV_MAX_TOKENS = 32
 STREAM_MAX_PAIRS_PER_SLOT = 75
 
 
-def layer_path(tokens: int, top_k: int, hidden: int, intermediate: int) -> int:
+def aligned16(*tensors: torch.Tensor) -> bool:
+    """Whether every tensor starts on a 16-byte boundary."""
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def layer_path(tokens: int, top_k: int, hidden: int, intermediate: int, *, aligned: bool = True) -> int:
     """The MLP path of a layer of `tokens` tokens with top_k pairs each: the
     decode GEMVs for a few tokens, the streaming MFMA kernel with partial sums
     (LMOE_PATH_STREAM, accumulation as accurate as the GEMVs') up to
     FUSED_DECODE_MAX_PAIRS pairs, the MFMA kernels past that.  The paths round
     differently, so the choice depends on nothing that changes when a layer is
     split into passes (slots, waves, routing).  The streaming kernel needs
-    hidden % 64 == 0; without it the GEMVs serve all of their range."""
+    hidden % 64 == 0 and hidden states and gate-up weights that start on 16-byte
+    boundaries (aligned); without them the GEMVs serve all of their range."""
     if tokens * top_k > FUSED_DECODE_MAX_PAIRS or intermediate > GEMV_MAX_I:
         return LMOE_PATH_MFMA
-    if tokens <= DECODE_GEMV_MAX_TOKENS or hidden % 64 != 0:
+    if tokens <= DECODE_GEMV_MAX_TOKENS or hidden % 64 != 0 or not aligned:
         return LMOE_PATH_GEMV
     return LMOE_PATH_STREAM
 
