@@ -174,6 +174,21 @@ def test_layer_path_depends_on_the_layer_only():
     assert pick(128, 512, h=1000) == native.MFMA_BLOCK_M
 
 
+def test_few_pairs_per_expert_keep_the_gemvs():
+    """Past the GEMVs' token count the line lies at a number of pairs per
+    expert of the layer: where the streaming kernel is the faster one with
+    every expert as likely.  Rows of other lengths have none."""
+    native = _native()
+    gemv, stream = native.LMOE_PATH_GEMV, native.LMOE_PATH_STREAM
+    path = native.layer_path
+    assert path(43, 8, 2048, 768, 128) == gemv and path(44, 8, 2048, 768, 128) == stream  # 344 and 352 pairs
+    assert path(33, 4, 2048, 1408, 60) == stream  # 2.2 pairs per expert
+    assert path(83, 4, 2048, 1408, 160) == gemv and path(84, 4, 2048, 1408, 160) == stream
+    assert path(33, 9, 7168, 2048, 257) == stream and path(33, 8, 1536, 768, 128) == stream
+    assert path(33, 1, 2048, 768, 1) == stream and path(32, 8, 2048, 768, 1) == gemv
+    assert path(129, 8, 2048, 768, 1024) == native.LMOE_PATH_MFMA  # past 1024 pairs whatever the experts
+
+
 def test_stream_two_passes_refuse_shapes_on_the_host():
     native = _native()
     lib = native.load_library()

@@ -34,3 +34,22 @@ def test_waves_of_few_experts_equal_the_full_layer(E, slots, T):
     assert len(report.waves) == E // slots
     assert torch.equal(dev.view(torch.int16), full.view(torch.int16))
     assert torch.equal(host.view(torch.int16), full.view(torch.int16))
+
+
+# the first and last token counts of either path at the line of 2.1 pairs per
+# expert of the layer (256 of them; a wave holds 64)
+@pytest.mark.parametrize("T", [67, 68])
+def test_waves_take_the_path_of_the_whole_layers_experts(T):
+    from vllm_moe_offload_amd import fused_moe, native
+
+    print(f"case waves at the line per expert T={T}", flush=True)
+    layer, rt, rng = _layer({}, E=256, slots=64)
+    dx = to_dev_bf16(normal_bf16(rng, (T, 1024), 1.0))
+    w, ids, _ = fused_moe.route(dx, layer.gate_weight, layer.router_spec)
+    kw = dict(layer_id=layer.layer_id, hidden=dx, topk_weights=w, topk_ids=ids, num_logical_experts=256)
+    path = native.layer_path(T, 8, 1024, 256, 256)
+    assert path == (native.LMOE_PATH_GEMV if T == 67 else native.LMOE_PATH_STREAM)
+    want = fused_moe.run_full_layer(rt, path=path, **kw).clone()
+    for out in (fused_moe.run_full_layer(rt, **kw), fused_moe.run_device_waves(rt, **kw),
+                fused_moe.run_wave_prefill(rt, **kw)[0]):
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16))

@@ -160,12 +160,20 @@ def fused_experts(
                              path=path, workspace=workspace)[0]
 
 
-def _layer_path(hidden, k: int, *w13) -> int:
-    """native.layer_path of a layer over the gate-up banks w13 (a pass's own
-    and, where there are several passes, all of them): one path for every
-    pass, so a split layer gives the unsplit layer's bits."""
+def _layer_path(hidden, k: int, n_experts: int, *w13) -> int:
+    """native.layer_path of a layer of n_experts experts (the length of its
+    slot table) over the gate-up banks w13 (a pass's own and, where there are
+    several passes, all of them): one path for every pass, so a split layer
+    gives the unsplit layer's bits."""
     T, H = hidden.shape
-    return native.layer_path(T, k, H, int(w13[0].shape[1]) // 2, aligned=native.aligned16(hidden, *w13))
+    return native.layer_path(T, k, H, int(w13[0].shape[1]) // 2, n_experts, aligned=native.aligned16(hidden, *w13))
+
+
+def _bank_layer_path(hidden, k: int, w13_slots, log2phy, overflow: PreparedSlotWeights | None) -> int:
+    """_layer_path of a layer run from one bank and, where it needs more
+    experts than that, an overflow buffer."""
+    n_experts = int(log2phy.numel()) if log2phy is not None else int(w13_slots.shape[0])
+    return _layer_path(hidden, k, n_experts, w13_slots, *([overflow.w1] if overflow is not None else []))
 
 
 def _overflow_perm(hidden, k: int, overflow: PreparedSlotWeights, ws: MoEWorkspace) -> native.Permutation:
@@ -251,7 +259,7 @@ def _fused_experts_ws(hidden, topk_weights, topk_ids, w13_slots, w2_slots, log2p
     ws = workspace or get_workspace(T, k, P, H, I, hidden.device)
     dst = out if out is not None else ws.out[:T]
     if path == native.LMOE_PATH_AUTO:
-        path = _layer_path(hidden, k, w13_slots, *([overflow.w1] if overflow is not None else []))
+        path = _bank_layer_path(hidden, k, w13_slots, log2phy, overflow)
     # the decode body; past its pair count path GEMV runs the two GEMVs apart
     decode = path == native.LMOE_PATH_GEMV and T * k <= native.FUSED_DECODE_MAX_PAIRS
     bm = _block_m(hidden, k, w13_slots, path)
@@ -349,7 +357,7 @@ def decode_layer(
         renormalize=bool(spec.renormalize), routed_scaling_factor=float(spec.routed_scaling_factor),
         n_shared=int(spec.n_shared), w_bf16=w_out, ids=ids_out, skip_unmapped=overflow is not None,
     )
-    path = _layer_path(hidden, kw, w13_slots, *([overflow.w1] if overflow is not None else []))
+    path = _bank_layer_path(hidden, kw, w13_slots, log2phy, overflow)
     bm = _block_m(hidden, kw, w13_slots, path)
     merged = overflow is not None and log2phy is not None and _merged_passes(hidden, kw, w13_slots, overflow, path)
     perm_b = None
@@ -662,10 +670,10 @@ def run_wave_prefill(
     profiling = bool(runtime.profile_path)
     wave_profiles: dict[int, dict] = {}
     ws = get_workspace(T, k, P, H, I, hidden.device, tag="waves")
-    mlp_path = _layer_path(hidden, k, bank.w13_slots) if path == native.LMOE_PATH_AUTO else path
     report = WaveRunReport(plan.waves, sched.compute_order)
     staged: dict[int, tuple] = {}
     total_logical = runtime.total_logical_expert_count_for_layer(layer_id=layer_id, fallback=num_logical_experts)
+    mlp_path = _layer_path(hidden, k, total_logical, bank.w13_slots) if path == native.LMOE_PATH_AUTO else path
     # pairs of a pinned shared suffix (ids in [routed, total)) run with the
     # first computed wave only; later waves' tables stop at the routed ids
     shared_pairs = phase_split.count_shared_suffix_pairs(topk_ids, routed, total_logical)
@@ -888,7 +896,7 @@ def run_device_waves(
             if isinstance(ev, torch.cuda.Event):
                 tx.wait_event(ev)
     released: list = [None] * len(stages)
-    mlp_path = _layer_path(hidden, k, bank.w13_slots) if path == native.LMOE_PATH_AUTO else path
+    mlp_path = _layer_path(hidden, k, total, bank.w13_slots) if path == native.LMOE_PATH_AUTO else path
     bm = _pass_block_m(P, H, I, dev, -(-(T * k) // n_waves), mlp_path)
     for w in range(n_waves):
         b = w % len(stages)

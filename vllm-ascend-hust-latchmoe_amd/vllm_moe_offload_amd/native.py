@@ -613,18 +613,33 @@ def _cu_count(device) -> int:
 _OFFSET32_LIMIT = 2**31 - 1
 
 
-# The decode GEMVs take a layer of up to this many tokens; past it the
-# weight-streaming MFMA kernel does.  A GEMV pays ~70 vector instructions per
-# row pair and token, the MFMA kernel has fewer bytes in flight per wave and a
-# longer chain before its first weight load.  gate-up + down, GEMV against
-# streaming (us; routing without and with the Zipf(1.1) rank bias):
-#   Qwen3 shape     16 tokens 111 / 119 and 72 / 70, 32: 159 / 171 and
-#                   102 / 94, 64: 202 / 183 and 167 / 130, 128: 280 / 197 and
-#                   257 / 169
-#   Qwen1.5-MoE     16 tokens 100 / 103 and 68 / 63, 32: 143 / 139 and
-#                   94 / 81, 48: 170 / 155 and 123 / 93
-#   DeepSeek-V3     8 tokens 712 / 718, 32: 2115 / 2099, 110: 3566 / 3134
+# The decode GEMVs take a layer of up to this many tokens, and past it one of
+# few pairs per expert; the rest goes to the weight-streaming MFMA kernel.  A
+# GEMV pays ~70 vector instructions per row pair and token, the MFMA kernel has
+# fewer bytes in flight per wave and a longer chain before its first weight
+# load, so the line lies at a number of pairs per expert, higher where the
+# GEMVs' rows fill the chunks that they are compiled for (GEMV_WHOLE_HIDDEN,
+# GEMV_WHOLE_INTERMEDIATE).  A layer's experts, GEMV / streaming, us, every
+# expert as likely (H, I, experts, top k):
+#   2048, 768, 128, 8     33 tokens 166 / 176, 40: 177 / 184, 44: 182 / 183, 64: 212 / 195
+#   2048, 768, 128, 4     33: 130 / 141, 64: 165 / 177, 80: 178 / 184
+#   2048, 1024, 128, 8    33: 220 / 239, 44: 243 / 247, 48: 248 / 250, 56: 265 / 255
+#   2048, 512, 256, 8     33: 166 / 183, 64: 224 / 238, 80: 246 / 253
+#   1024, 512, 128, 8     33: 67 / 74, 44: 71 / 76, 56: 77 / 78
+#   4096, 768, 128, 8     33: 326 / 340, 40: 352 / 351, 48: 372 / 356
+#   2048, 1408, 60, 4     28: 143 / 143, 33: 151 / 149, 48: 174 / 162
+#   2048, 1408, 160, 4    33: 243 / 259, 64: 329 / 344
+#   4096, 1536, 64, 4     33: 333 / 345, 40: 347 / 347, 64: 417 / 363
+#   5120, 1536, 256, 8    33: 1138 / 1131, 64: 1609 / 1527
+#   7168, 2048, 257, 9    8 tokens 712 / 718, 32: 2115 / 2099, 110: 3566 / 3134
+# Skewed routing has fewer experts at work and moves the line down, but is not
+# known when the layer is launched: with the Zipf(1.1) rank bias the first of
+# these takes 107 / 100 at 33 tokens (whole step) and 128 / 109 at 44.
 DECODE_GEMV_MAX_TOKENS = 32
+GEMV_MAX_PAIRS_PER_EXPERT = 2.1
+GEMV_MAX_PAIRS_PER_EXPERT_WHOLE = 2.75
+GEMV_WHOLE_HIDDEN = (1024, 2048, 4096)
+GEMV_WHOLE_INTERMEDIATE = (512, 768, 1024, 2048, 4096)
 # Most pairs per slot, on average, of a pass on STREAM_BLOCK_M-row tiles: past
 # one tile per slot the second one costs as much as the wider tiles do.
 # Streaming against the 320-row tiles (us): Qwen3 shape 1024 tokens (64 pairs
@@ -644,9 +659,11 @@ def aligned16(*tensors: torch.Tensor) -> bool:
     return all(t.data_ptr() % 16 == 0 for t in tensors)
 
 
-def layer_path(tokens: int, top_k: int, hidden: int, intermediate: int, *, aligned: bool = True) -> int:
-    """The MLP path of a layer of `tokens` tokens with top_k pairs each: the
-    decode GEMVs for a few tokens, the streaming MFMA kernel with partial sums
+def layer_path(tokens: int, top_k: int, hidden: int, intermediate: int, n_experts: int | None = None, *,
+               aligned: bool = True) -> int:
+    """The MLP path of a layer of `tokens` tokens with top_k pairs each over
+    n_experts experts (all of the layer's, also where a pass holds fewer): the
+    decode GEMVs for a few tokens or few pairs per expert, the streaming MFMA kernel with partial sums
     (LMOE_PATH_STREAM, accumulation as accurate as the GEMVs') up to
     FUSED_DECODE_MAX_PAIRS pairs, the MFMA kernels past that.  The paths round
     differently, so the choice depends on nothing that changes when a layer is
@@ -657,6 +674,10 @@ def layer_path(tokens: int, top_k: int, hidden: int, intermediate: int, *, align
         return LMOE_PATH_MFMA
     if tokens <= DECODE_GEMV_MAX_TOKENS or hidden % 64 != 0 or not aligned:
         return LMOE_PATH_GEMV
+    if n_experts is not None and hidden in GEMV_WHOLE_HIDDEN:
+        most = GEMV_MAX_PAIRS_PER_EXPERT_WHOLE if intermediate in GEMV_WHOLE_INTERMEDIATE else GEMV_MAX_PAIRS_PER_EXPERT
+        if tokens * top_k < most * n_experts:
+            return LMOE_PATH_GEMV
     return LMOE_PATH_STREAM
 
 
