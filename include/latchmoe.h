@@ -317,6 +317,17 @@ int lmoe_grouped_mlp(const void* x, int T, int H, int I, int k,
                      const int32_t* meta, int n_pairs, int block_m, int path,
                      void* act, void* y, hipStream_t stream);
 
+/* lmoe_grouped_mlp of a pass that is expected to place only pass_pairs of the
+ * n_pairs pairs (a wave of a layer past its slot bank): the kernel's form is
+ * chosen for pass_pairs, every buffer and bound is that of n_pairs.  The same
+ * bits whatever pass_pairs is; negative: LMOE_ERR_ARG. */
+int lmoe_grouped_mlp_pass(const void* x, int T, int H, int I, int k,
+                          const void* w13_slots, const void* w2_slots, int n_slots,
+                          const int32_t* offsets, const int32_t* sorted_pairs,
+                          const int32_t* active, const int32_t* tile_off,
+                          const int32_t* meta, int n_pairs, int pass_pairs, int block_m,
+                          int path, void* act, void* y, hipStream_t stream);
+
 /* The two halves of lmoe_grouped_mlp, callable on their own (same argument
  * meaning): GMM1 + SwiGLU into act, and GMM2 from act into y.  Replace the
  * separate npu_grouped_matmul + npu_swiglu and npu_grouped_matmul calls of

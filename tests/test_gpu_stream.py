@@ -189,6 +189,22 @@ def test_few_pairs_per_expert_keep_the_gemvs():
     assert path(129, 8, 2048, 768, 1024) == native.LMOE_PATH_MFMA  # past 1024 pairs whatever the experts
 
 
+def test_pass_pairs_choose_the_tiles_and_n_pairs_bound_the_offsets():
+    native = _native()
+    pick = lambda n, p=None, h=2048: native.prefill_block_m(64, h, 768, cu_count=256, n_pairs=n, pass_pairs=p)
+    assert pick(9600) == native.PART_BLOCK_M and pick(9600, 4800) == native.STREAM_BLOCK_M
+    assert pick(9600, 4801) == native.PART_BLOCK_M
+    # a wave's kernels address rows of the whole layer's buffers
+    assert pick(2**20 + 1, 4800) == native.MFMA_BLOCK_M
+    import ctypes
+
+    p = ctypes.c_void_p(4096)
+    lib = native.load_library()
+    args = (p, 64, 2048, 768, 8, p, p, 8, p, p, p, p, p, 512)
+    assert lib.lmoe_grouped_mlp_pass(*args, -1, 96, native.LMOE_PATH_MFMA, p, p, None) == native.LMOE_ERR_ARG
+    assert lib.lmoe_grouped_mlp_pass(*args[:13], 0, 0, 96, native.LMOE_PATH_MFMA, p, p, None) == 0
+
+
 def test_stream_two_passes_refuse_shapes_on_the_host():
     native = _native()
     lib = native.load_library()

@@ -53,3 +53,36 @@ def test_waves_take_the_path_of_the_whole_layers_experts(T):
     for out in (fused_moe.run_full_layer(rt, **kw), fused_moe.run_device_waves(rt, **kw),
                 fused_moe.run_wave_prefill(rt, **kw)[0]):
         assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+
+
+def test_waves_take_the_row_tiles_of_their_own_pairs(monkeypatch):
+    """384 pairs of 3072 in a wave of 8 slots: 48 per slot, the 96-row tiles,
+    by host- and device-planned waves alike; the bits are those of the 320-row
+    tiles, which 384 per slot would take."""
+    from vllm_moe_offload_amd import fused_moe, native
+
+    T = 384
+    print(f"case row tiles of waves T={T}", flush=True)
+    layer, rt, rng = _layer({}, E=64, slots=8)
+    dx = to_dev_bf16(normal_bf16(rng, (T, 1024), 1.0))
+    w, ids, _ = fused_moe.route(dx, layer.gate_weight, layer.router_spec)
+    kw = dict(layer_id=layer.layer_id, hidden=dx, topk_weights=w, topk_ids=ids, num_logical_experts=64)
+    seen, permute, mlp = [], native.permute, native.grouped_mlp
+
+    def outs():
+        return [f.clone() for f in (fused_moe.run_device_waves(rt, **kw), fused_moe.run_wave_prefill(rt, **kw)[0])]
+
+    monkeypatch.setattr(native, "permute", lambda *a, **k: (seen.append(k["block_m"]), permute(*a, **k))[1])
+    got = outs()
+    assert seen == [native.STREAM_BLOCK_M] * 16
+    monkeypatch.setattr(native, "STREAM_MAX_PAIRS_PER_SLOT", 0)
+    want = outs()
+    assert set(seen[16:]) == {native.PART_BLOCK_M}
+    monkeypatch.undo()
+    # the kernel's form is chosen by the pass's pairs: none, and all of them
+    for pairs in (0, T * 8):
+        monkeypatch.setattr(native, "grouped_mlp", lambda *a, **k: mlp(*a, **{**k, "pass_pairs": pairs}))
+        got += outs()
+    for out in got:
+        assert torch.equal(out.view(torch.int16), want[0].view(torch.int16))
+    assert torch.equal(want[0], want[1])

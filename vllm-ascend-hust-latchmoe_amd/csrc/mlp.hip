@@ -927,9 +927,11 @@ static bool part_offsets_fit(const GemmArgs& g, int n_pairs) {
 constexpr long long kStreamWideBlocks = 1500;
 constexpr int kStreamWiderRows = 40;
 
+// pass_pairs: the pairs expected in the pass, for the choice of its form (n_pairs
+// bounds the grid: a wave of a layer holds a part of them).
 template <int MODE, bool SPLIT, bool TWO>
-static int launch_stream(const StreamArgs& a, const StreamArgs& b, int n_pairs, int max_active,
-                         hipStream_t stream) {
+static int launch_stream(const StreamArgs& a, const StreamArgs& b, int n_pairs, int pass_pairs,
+                         int max_active, hipStream_t stream) {
   if (a.K % 64 != 0 || a.N % 64 != 0) return LMOE_ERR_SHAPE;
   const long long tiles = n_pairs / kStreamBM + static_cast<long long>(max_active);
   if (tiles > 65535) return LMOE_ERR_SHAPE;
@@ -944,7 +946,7 @@ static int launch_stream(const StreamArgs& a, const StreamArgs& b, int n_pairs, 
     // fewer rows it is slower (128 of 19: 145 -> 157; 257 of 10: 2294 -> 2345),
     // and the down GEMM (more output rows to store) gains nothing.
     const int wider = (a.N + 2 * wide_cols - 1) / (2 * wide_cols);
-    if (n_pairs >= kStreamWiderRows * static_cast<long long>(a.P) &&
+    if (pass_pairs >= kStreamWiderRows * static_cast<long long>(a.P) &&
         static_cast<long long>(wider) * max_active >= 512) {
       hipLaunchKernelGGL((stream_gemm_kernel<MODE, 4, SPLIT, TWO>),
                          dim3(wider, static_cast<unsigned>(tiles)), dim3(kStreamWaves * 64), 0,
@@ -965,15 +967,15 @@ static int launch_stream(const StreamArgs& a, const StreamArgs& b, int n_pairs, 
 
 // split: LMOE_PATH_STREAM
 template <int MODE, bool TWO>
-static int launch_stream(const StreamArgs& a, const StreamArgs& b, int n_pairs, int max_active,
-                         bool split, hipStream_t stream) {
-  return split ? launch_stream<MODE, true, TWO>(a, b, n_pairs, max_active, stream)
-               : launch_stream<MODE, false, TWO>(a, b, n_pairs, max_active, stream);
+static int launch_stream(const StreamArgs& a, const StreamArgs& b, int n_pairs, int pass_pairs,
+                         int max_active, bool split, hipStream_t stream) {
+  return split ? launch_stream<MODE, true, TWO>(a, b, n_pairs, pass_pairs, max_active, stream)
+               : launch_stream<MODE, false, TWO>(a, b, n_pairs, pass_pairs, max_active, stream);
 }
 
 template <int MODE>
-static int launch_grouped_mfma(GemmArgs g, int n_pairs, int max_active, int block_m, int path,
-                               hipStream_t stream) {
+static int launch_grouped_mfma(GemmArgs g, int n_pairs, int pass_pairs, int max_active,
+                               int block_m, int path, hipStream_t stream) {
   if (path == LMOE_PATH_STREAM && block_m != kStreamBM) return LMOE_ERR_UNSUPPORTED;
   if (block_m != PartTile::BM && block_m != PrefillTile::BM && block_m != kBM &&
       block_m != kStreamBM)
@@ -987,7 +989,8 @@ static int launch_grouped_mfma(GemmArgs g, int n_pairs, int max_active, int bloc
     if (!part_offsets_fit<MODE>(g, n_pairs)) return LMOE_ERR_SHAPE;  // take block_m 256
     const StreamArgs a{g.a, g.w, g.w_slot_stride, g.N, g.K, g.topk, g.P, g.offsets, g.sorted_pairs,
                        g.tile_off, g.meta, static_cast<uint16_t*>(g.out)};
-    return launch_stream<MODE, false>(a, a, n_pairs, max_active, path == LMOE_PATH_STREAM, stream);
+    return launch_stream<MODE, false>(a, a, n_pairs, pass_pairs, max_active,
+                                      path == LMOE_PATH_STREAM, stream);
   }
   if (block_m == PartTile::BM) {
     if (g.K % PartTile::BK != 0 || g.N % 8 != 0) return LMOE_ERR_SHAPE;
@@ -1029,12 +1032,11 @@ static int resolve_path(int path, int n_pairs) {
   return path == LMOE_PATH_AUTO ? (n_pairs <= 256 ? LMOE_PATH_GEMV : LMOE_PATH_MFMA) : path;
 }
 
-extern "C" int lmoe_gateup_silu(const void* x, int T, int H, int I, int k,
-                                const void* w13_slots, int n_slots,
-                                const int32_t* offsets, const int32_t* sorted_pairs,
-                                const int32_t* active, const int32_t* tile_off,
-                                const int32_t* meta, int n_pairs, int block_m,
-                                int path, void* act, hipStream_t stream) {
+static int gateup_silu_impl(const void* x, int T, int H, int I, int k, const void* w13_slots,
+                            int n_slots, const int32_t* offsets, const int32_t* sorted_pairs,
+                            const int32_t* active, const int32_t* tile_off, const int32_t* meta,
+                            int n_pairs, int pass_pairs, int block_m, int path, void* act,
+                            hipStream_t stream) {
   int st = check_mlp_args(T, H, I, k, n_slots, n_pairs);
   if (st != LMOE_OK) return st;
   if (n_pairs == 0) return LMOE_OK;  // an empty batch: nothing read or written
@@ -1069,9 +1071,19 @@ extern "C" int lmoe_gateup_silu(const void* x, int T, int H, int I, int k,
   g.K = H;
   g.I = I;
   g.out = act;
-  st = launch_grouped_mfma<kGateUp>(g, n_pairs, max_active, block_m, path, stream);
+  st = launch_grouped_mfma<kGateUp>(g, n_pairs, pass_pairs, max_active, block_m, path, stream);
   if (st != LMOE_OK) return st;
   LMOE_RETURN_LAUNCH();
+}
+
+extern "C" int lmoe_gateup_silu(const void* x, int T, int H, int I, int k,
+                                const void* w13_slots, int n_slots,
+                                const int32_t* offsets, const int32_t* sorted_pairs,
+                                const int32_t* active, const int32_t* tile_off,
+                                const int32_t* meta, int n_pairs, int block_m,
+                                int path, void* act, hipStream_t stream) {
+  return gateup_silu_impl(x, T, H, I, k, w13_slots, n_slots, offsets, sorted_pairs, active,
+                          tile_off, meta, n_pairs, n_pairs, block_m, path, act, stream);
 }
 
 extern "C" int lmoe_down(const void* act, int H, int I, const void* w2_slots, int n_slots,
@@ -1112,9 +1124,29 @@ extern "C" int lmoe_down(const void* act, int H, int I, const void* w2_slots, in
   g.N = H;
   g.K = I;
   g.out = yb;
-  st = launch_grouped_mfma<kDown>(g, n_pairs, max_active, block_m, path, stream);
+  st = launch_grouped_mfma<kDown>(g, n_pairs, n_pairs, max_active, block_m, path, stream);
   if (st != LMOE_OK) return st;
   LMOE_RETURN_LAUNCH();
+}
+
+extern "C" int lmoe_grouped_mlp_pass(const void* x, int T, int H, int I, int k,
+                                     const void* w13_slots, const void* w2_slots,
+                                     int n_slots, const int32_t* offsets,
+                                     const int32_t* sorted_pairs,
+                                     const int32_t* active, const int32_t* tile_off,
+                                     const int32_t* meta, int n_pairs, int pass_pairs,
+                                     int block_m, int path, void* act, void* y,
+                                     hipStream_t stream) {
+  int st = check_mlp_args(T, H, I, k, n_slots, n_pairs);
+  if (st != LMOE_OK) return st;
+  if (pass_pairs < 0) return LMOE_ERR_ARG;
+  if (n_pairs == 0) return LMOE_OK;
+  if (w2_slots == nullptr || y == nullptr) return LMOE_ERR_ARG;
+  st = gateup_silu_impl(x, T, H, I, k, w13_slots, n_slots, offsets, sorted_pairs, active,
+                        tile_off, meta, n_pairs, pass_pairs, block_m, path, act, stream);
+  if (st != LMOE_OK) return st;
+  return lmoe_down(act, H, I, w2_slots, n_slots, offsets, sorted_pairs, active, tile_off, meta,
+                   n_pairs, block_m, path, y, stream);
 }
 
 extern "C" int lmoe_grouped_mlp(const void* x, int T, int H, int I, int k,
@@ -1125,15 +1157,9 @@ extern "C" int lmoe_grouped_mlp(const void* x, int T, int H, int I, int k,
                                 const int32_t* meta, int n_pairs, int block_m,
                                 int path, void* act, void* y,
                                 hipStream_t stream) {
-  int st = check_mlp_args(T, H, I, k, n_slots, n_pairs);
-  if (st != LMOE_OK) return st;
-  if (n_pairs == 0) return LMOE_OK;
-  if (w2_slots == nullptr || y == nullptr) return LMOE_ERR_ARG;
-  st = lmoe_gateup_silu(x, T, H, I, k, w13_slots, n_slots, offsets, sorted_pairs, active,
-                            tile_off, meta, n_pairs, block_m, path, act, stream);
-  if (st != LMOE_OK) return st;
-  return lmoe_down(act, H, I, w2_slots, n_slots, offsets, sorted_pairs, active, tile_off, meta,
-                   n_pairs, block_m, path, y, stream);
+  return lmoe_grouped_mlp_pass(x, T, H, I, k, w13_slots, w2_slots, n_slots, offsets, sorted_pairs,
+                               active, tile_off, meta, n_pairs, n_pairs, block_m, path, act, y,
+                               stream);
 }
 
 extern "C" int lmoe_decode_mlp_two_passes(
@@ -1241,13 +1267,13 @@ extern "C" int lmoe_stream_mlp_two_passes(
   const StreamArgs gb{xb, static_cast<const uint16_t*>(w13_b), slot_elems_w13(H, I), I, H, k,
                       n_slots_b, offsets_b, sorted_pairs_b, tile_off_b, meta_b, actb};
   const bool split = path == LMOE_PATH_STREAM;
-  st = launch_stream<kGateUp, true>(ga, gb, n_pairs, max_active, split, stream);
+  st = launch_stream<kGateUp, true>(ga, gb, n_pairs, n_pairs, max_active, split, stream);
   if (st != LMOE_OK) return st;
   const StreamArgs da{actb, static_cast<const uint16_t*>(w2_a), slot_elems_w2(H, I), H, I, 1,
                       n_slots_a, offsets_a, sorted_pairs_a, tile_off_a, meta_a, yb};
   const StreamArgs db{actb, static_cast<const uint16_t*>(w2_b), slot_elems_w2(H, I), H, I, 1,
                       n_slots_b, offsets_b, sorted_pairs_b, tile_off_b, meta_b, yb};
-  st = launch_stream<kDown, true>(da, db, n_pairs, max_active, split, stream);
+  st = launch_stream<kDown, true>(da, db, n_pairs, n_pairs, max_active, split, stream);
   if (st != LMOE_OK) return st;
   LMOE_RETURN_LAUNCH();
 }

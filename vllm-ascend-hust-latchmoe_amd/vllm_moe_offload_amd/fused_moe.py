@@ -181,15 +181,15 @@ def _overflow_perm(hidden, k: int, overflow: PreparedSlotWeights, ws: MoEWorkspa
     return ws.overflow_perm(hidden.shape[0] * k, int(overflow.physical_expert_count), hidden.device)
 
 
-def _pass_block_m(n_experts: int, H: int, I: int, device, n_pairs: int, path: int) -> int:
+def _pass_block_m(n_experts: int, H: int, I: int, device, n_pairs: int, path: int, pass_pairs: int | None = None) -> int:
     """The row-tile height to build the permutation of a pass over n_experts
     slots with: the path's own (the GEMVs read no tile table, path STREAM has
-    one height), else the MFMA kernel's for n_pairs pairs."""
+    one height), else the MFMA kernel's for pass_pairs of n_pairs pairs."""
     if path == native.LMOE_PATH_GEMV:
         return native.MFMA_BLOCK_M
     if path == native.LMOE_PATH_STREAM:
         return native.STREAM_BLOCK_M
-    return native.prefill_block_m(n_experts, H, I, device, n_pairs=n_pairs)
+    return native.prefill_block_m(n_experts, H, I, device, n_pairs=n_pairs, pass_pairs=pass_pairs)
 
 
 def _block_m(hidden, k: int, w13_slots, path: int) -> int:
@@ -718,13 +718,14 @@ def run_wave_prefill(
             runtime.wait_prefill_stage_plan(ready)
             t_mlp = perf_counter()
             handle = runtime.begin_slot_compute(prepared)
+            pairs = plan.wave_tokens(plan.waves[w]) + (shared_pairs if first else 0)
             try:
                 native.permute(topk_ids, ws.perm, log2phy=prepared.log2phy, skip_unmapped=True, keep_rows=not first,
                                table_len=total_logical if first else routed,
-                               block_m=_pass_block_m(len(plan.waves[w]), H, I, hidden.device, T * k, mlp_path))
+                               block_m=_pass_block_m(len(plan.waves[w]), H, I, hidden.device, T * k, mlp_path, pairs))
                 first = False
                 native.grouped_mlp(hidden, k, prepared.w1, prepared.w2, ws.perm, ws.act[: T * k], ws.y[: T * k],
-                                   path=mlp_path)
+                                   path=mlp_path, pass_pairs=pairs)
             finally:
                 runtime.end_slot_compute(handle)
             if buf is not None:
@@ -897,7 +898,8 @@ def run_device_waves(
                 tx.wait_event(ev)
     released: list = [None] * len(stages)
     mlp_path = _layer_path(hidden, k, total, bank.w13_slots) if path == native.LMOE_PATH_AUTO else path
-    bm = _pass_block_m(P, H, I, dev, -(-(T * k) // n_waves), mlp_path)
+    pairs = -(-(T * k) // n_waves)  # of a wave, on average
+    bm = _pass_block_m(P, H, I, dev, T * k, mlp_path, pairs)
     for w in range(n_waves):
         b = w % len(stages)
         stage, table = stages[b], tables[b]
@@ -912,7 +914,7 @@ def run_device_waves(
         compute.wait_event(ready)
         native.permute(topk_ids, ws.perm, log2phy=table, skip_unmapped=True, keep_rows=w > 0, block_m=bm)
         native.grouped_mlp(hidden, k, stage.w13_slots, stage.w2_slots, ws.perm, ws.act[: T * k], ws.y[: T * k],
-                           path=mlp_path)
+                           path=mlp_path, pass_pairs=pairs)
         done = torch.cuda.Event()
         done.record(compute)
         released[b] = done

@@ -56,6 +56,7 @@ EXPORTED_SYMBOLS = (
     "lmoe_permute_two_tables",
     "lmoe_gather_rows",
     "lmoe_grouped_mlp",
+    "lmoe_grouped_mlp_pass",
     "lmoe_gateup_silu",
     "lmoe_down",
     "lmoe_decode_mlp_two_passes",
@@ -116,6 +117,10 @@ _SIGNATURES = {
     "lmoe_grouped_mlp": (
         _i,
         [_vp, _i, _i, _i, _i, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _vp, _vp],
+    ),
+    "lmoe_grouped_mlp_pass": (
+        _i,
+        [_vp, _i, _i, _i, _i, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp, _vp],
     ),
     "lmoe_gateup_silu": (
         _i,
@@ -682,12 +687,14 @@ def layer_path(tokens: int, top_k: int, hidden: int, intermediate: int, n_expert
 
 
 def prefill_block_m(n_experts: int, hidden: int, intermediate: int, device="cuda",
-                    cu_count: int | None = None, n_pairs: int | None = None) -> int:
+                    cu_count: int | None = None, n_pairs: int | None = None,
+                    pass_pairs: int | None = None) -> int:
     """Row-tile height for the prefill GEMMs of one pass over n_experts slots
-    (the block_m to build the permutation with).
+    (the block_m to build the permutation with).  n_pairs is the layer's pair
+    count, pass_pairs the pass's own where that is one wave of the layer.
 
-    STREAM_BLOCK_M selects the weight-streaming kernel, for passes of few pairs per slot
-    (n_pairs over n_experts, when n_pairs is given).
+    STREAM_BLOCK_M selects the weight-streaming kernel, for passes of few pairs
+    per slot (pass_pairs over n_experts, when n_pairs is given).
 
     320 selects the kernel with one workgroup per CU: a slot of up to 320
     pairs is one row tile, and each CU runs an equal number of units (a row
@@ -704,8 +711,9 @@ def prefill_block_m(n_experts: int, hidden: int, intermediate: int, device="cuda
         return MFMA_BLOCK_M
     if n_pairs is not None and int(n_pairs) * max(int(hidden), int(intermediate)) > _OFFSET32_LIMIT:
         return MFMA_BLOCK_M
-    if n_pairs is not None and int(n_pairs) <= STREAM_MAX_PAIRS_PER_SLOT * int(n_experts):
-        return STREAM_BLOCK_M
+    if n_pairs is not None:
+        if int(n_pairs if pass_pairs is None else pass_pairs) <= STREAM_MAX_PAIRS_PER_SLOT * int(n_experts):
+            return STREAM_BLOCK_M
     cus = int(cu_count) if cu_count is not None else _cu_count(device)
     units = int(n_experts) * ((int(intermediate) + 127) // 128)
     if cus < units <= cus + cus // 4:
@@ -892,9 +900,12 @@ def grouped_mlp(
     y: torch.Tensor,
     *,
     path: int = LMOE_PATH_AUTO,
+    pass_pairs: int | None = None,
     stream=None,
 ) -> torch.Tensor:
-    """y[pair] = W2_s . (silu(W13_s[:I] x) * W13_s[I:] x) for the placed pairs."""
+    """y[pair] = W2_s . (silu(W13_s[:I] x) * W13_s[I:] x) for the placed pairs.
+    pass_pairs: how many of the pairs the pass is expected to place, where it
+    is one wave of its layer (chooses the kernel's form, not its bits)."""
     lib = load_library()
     _need(x, "x", torch.bfloat16)
     T, H = x.shape
@@ -906,13 +917,13 @@ def grouped_mlp(
     _need(act, "act", torch.bfloat16, (perm.n_pairs, I))
     _need(y, "y", torch.bfloat16, (perm.n_pairs, H))
     _check(
-        lib.lmoe_grouped_mlp(
+        lib.lmoe_grouped_mlp_pass(
             _ptr(x), T, H, I, int(top_k), _ptr(w13_slots), _ptr(w2_slots), P,
             _ptr(perm.offsets), _ptr(perm.sorted_pairs), _ptr(perm.active), _ptr(perm.tile_off),
-            _ptr(perm.meta), perm.n_pairs, perm.block_m, int(path), _ptr(act), _ptr(y),
-            _stream(stream),
+            _ptr(perm.meta), perm.n_pairs, perm.n_pairs if pass_pairs is None else int(pass_pairs), perm.block_m,
+            int(path), _ptr(act), _ptr(y), _stream(stream),
         ),
-        "lmoe_grouped_mlp",
+        "lmoe_grouped_mlp_pass",
     )
     return y
 
