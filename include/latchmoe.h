@@ -413,15 +413,15 @@ int lmoe_down_combine(const void* act, int T, int H, int I, int k,
  * the rest, which give the same out bit for bit:
  *   the down GEMV fused with the weighted combine, every workgroup walking the
  *   slots for a few output columns of every token (T*k <= 16, or y == NULL);
- *   for 2 and more tokens of up to 256 pairs with 256 < I <= 1024 and
- *   1792 <= H <= 2048 or 896 <= H <= 1024 (one workgroup per CU), the same in
- *   a form that streams the slots' rows without a gap;
+ *   for 2 and more tokens of up to 256 pairs with 256 < I <= 1024 where H / 8
+ *   (H / 4 for H <= 1024) workgroups are 7/8 of the CUs to all of them (on 256
+ *   CUs 1792 <= H <= 2048 and 896 <= H <= 1024), the same in a form that
+ *   streams the slots' rows without a gap;
  *   for more than 16 pairs with a y workspace, else, the down GEMV per (row
  *   block, slot) into y and the combine (three launches).
  * With more than 16 pairs y, where given, holds the [T*k, H] bf16 down rows in
  * flat pair order on return.  Each slot's weights are read once however many
- * tokens chose
- * it.  distinct_slots != 0 promises that no slot serves two pairs of one
+ * tokens chose it.  distinct_slots != 0 promises that no slot serves two pairs of one
  * token (true for ids from the routers, which pick distinct experts, through
  * a slot table, which maps distinct experts to distinct slots); with one
  * token it selects kernels that take active rank a as sorted position a.

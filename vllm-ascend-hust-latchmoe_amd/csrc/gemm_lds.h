@@ -358,6 +358,20 @@ __global__ __launch_bounds__(C::THREADS) void grouped_gemm_lds_kernel(GemmArgs g
   }
 }
 
+// CUs of the current device, queried once per device.
+static int device_cus() {
+  static int cached[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 256;
+  if (dev < 64 && cached[dev] > 0) return cached[dev];
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      cus <= 0)
+    cus = 256;
+  if (dev < 64) cached[dev] = cus;
+  return cus;
+}
+
 // Upper bound on launched workgroups for up to ub_tiles row tiles: the grid
 // is a multiple of 8 with ceil(items / 8) workgroups per XCD.
 __host__ inline int lds_gemm_grid(int ub_tiles, int n_col_tiles) {

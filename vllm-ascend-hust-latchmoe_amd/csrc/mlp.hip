@@ -834,7 +834,7 @@ static int launch_down_rows(const uint16_t* act, int H, int I, const uint16_t* w
 
 // down_combine_few_kernel serves 2 and more tokens of up to kFewPairs pairs
 // where 8 or (H <= 1024) 4 output columns per block make one block for nearly
-// every CU (224 to 256 of them): its waves stream a CU's whole share of W2
+// every CU (7/8 of them to all: 224 to 256 of 256): its waves stream a CU's whole share of W2
 // from start to end; bound by the weights' stream.  Decode body, separate
 // kernels -> this one (us, 2 / 8 / 32 tokens; y given, its store is up to 1 us):
 //   128 experts, top 8, H 2048, I 768   26.8 / 52.6 / 103.9 -> 24.7 / 50.8 / 102.2
@@ -847,7 +847,9 @@ static int launch_down_rows(const uint16_t* act, int H, int I, const uint16_t* w
 // I > 1024 needs two rows per half wave (I 1408, 24 tokens 87 -> 98).
 static bool down_combine_few_fits(int T, int n_pairs, int H, int I) {
   const int blocks = H <= 1024 ? (H + 3) / 4 : (H + 7) / 8;
-  return T > 1 && n_pairs <= kFewPairs && I > 256 && I <= 1024 && blocks >= 224 && blocks <= 256;
+  const int cus = device_cus();
+  return T > 1 && n_pairs <= kFewPairs && I > 256 && I <= 1024 && 8 * blocks >= 7 * cus &&
+         blocks <= cus;
 }
 
 static void launch_down_combine_few(const uint16_t* act, int T, int H, int I, int k,
@@ -892,20 +894,8 @@ static void launch_combine(const uint16_t* y, const int32_t* row_idx, const uint
 using PrefillTile = LdsTile<256, 256, 2, 4, 2>;
 
 // Workgroups of the block-range kernel: one per CU, a multiple of 8 (one
-// share per XCD), queried once per device.
-static int part_grid() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 256;
-  if (dev < 64 && cached[dev] > 0) return cached[dev];
-  int cus = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      cus <= 0)
-    cus = 256;
-  const int grid = ((cus + 7) / 8) * 8;
-  if (dev < 64) cached[dev] = grid;
-  return grid;
-}
+// share per XCD).
+static int part_grid() { return (device_cus() + 7) / 8 * 8; }
 
 // The block-range kernel forms operand offsets in 32 bits: activation row r
 // starts at r * K, the rows read are token rows (gate-up: sorted pair / topk
@@ -921,10 +911,10 @@ static bool part_offsets_fit(const GemmArgs& g, int n_pairs) {
 }
 
 // The wide form (two weight tiles per wave) once its blocks fill the CUs about
-// twice over at three per CU, else the narrow one, whose twice as many blocks
+// twice over at three per CU (1500 blocks on 256), else the narrow one, whose twice as many blocks
 // even out the last round: 128 slots of the Qwen3 shape 182 us wide against
 // 190 narrow, 64 slots at 40 tokens 123 against 113 (gate-up + down).
-constexpr long long kStreamWideBlocks = 1500;
+constexpr long long kStreamWideBlocks = 1500;  // per 256 CUs
 constexpr int kStreamWiderRows = 40;
 
 // pass_pairs: the pairs expected in the pass, for the choice of its form (n_pairs
@@ -947,14 +937,14 @@ static int launch_stream(const StreamArgs& a, const StreamArgs& b, int n_pairs, 
     // and the down GEMM (more output rows to store) gains nothing.
     const int wider = (a.N + 2 * wide_cols - 1) / (2 * wide_cols);
     if (pass_pairs >= kStreamWiderRows * static_cast<long long>(a.P) &&
-        static_cast<long long>(wider) * max_active >= 512) {
+        static_cast<long long>(wider) * max_active >= 2 * device_cus()) {
       hipLaunchKernelGGL((stream_gemm_kernel<MODE, 4, SPLIT, TWO>),
                          dim3(wider, static_cast<unsigned>(tiles)), dim3(kStreamWaves * 64), 0,
                          stream, a, b, n_pairs);
       return LMOE_OK;
     }
   }
-  if (static_cast<long long>(wide) * max_active >= kStreamWideBlocks)
+  if (256LL * wide * max_active >= kStreamWideBlocks * device_cus())
     hipLaunchKernelGGL((stream_gemm_kernel<MODE, 2, SPLIT, TWO>),
                        dim3(wide, static_cast<unsigned>(tiles)), dim3(kStreamWaves * 64), 0, stream,
                        a, b, n_pairs);

@@ -33,7 +33,6 @@ constexpr int kOneTokenRouterThreads = 512;
 // 7168 x 256 58 against 63.
 using DenseGateTile = LdsTile<64, 64, 2, 2, 6>;
 using DenseGateWideTile = LdsTile<64, 128, 1, 2, 4>;
-constexpr int kDenseGateTiles = 256;  // tiles of one round of the CUs
 constexpr int kGateTok = 4;         // tokens per reduction in the gate GEMV
 // one-launch router: tagged logit words from int32 offset 64 of sync (256
 // bytes past the arrival counter), and the re-reads of a stale word

@@ -82,7 +82,7 @@ extern "C" int lmoe_router_gate(const void* x, const void* wg, int T, int H,
       using C = decltype(tile);
       return lds_gemm_grid((T + C::BM - 1) / C::BM, (E + C::BN - 1) / C::BN);
     };
-    if (tiles(DenseGateTile{}) <= kDenseGateTiles)
+    if (tiles(DenseGateTile{}) <= device_cus())
       hipLaunchKernelGGL((grouped_gemm_lds_kernel<kDense, DenseGateTile>),
                          dim3(tiles(DenseGateTile{})), dim3(DenseGateTile::THREADS), 0, stream, g);
     else
