@@ -185,9 +185,7 @@ __global__ __launch_bounds__(C::THREADS) void grouped_gemm_lds_kernel(GemmArgs g
   const int rot = C::BK == 64 ? k_phase<MODE>(n0, KT) : 0;
   auto issue = [&](int kt, int buf) {
     char* st = smem + buf * C::STAGE_BYTES;
-    int kr = kt + rot;
-    if (kr >= KT) kr -= KT;
-    const int koff = kr * C::BK;
+    const int koff = k_step<MODE>(kt, rot, KT) * C::BK;
 #pragma unroll
     for (int q = 0; q < C::QA; ++q) load_lds16(a_src[q] + koff, st + (wave * C::QA + q) * 1024);
 #pragma unroll

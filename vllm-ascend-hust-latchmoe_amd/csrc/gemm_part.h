@@ -166,9 +166,7 @@ __device__ __forceinline__ void part_unit(const GemmArgs& g, char* smem, int* s_
 
   auto issue = [&](int kt, int buf) {
     char* st = smem + buf * S::STAGE_BYTES;
-    int kr = kt + rot;
-    if (kr >= KT) kr -= KT;
-    const int koff = kr * S::BK;
+    const int koff = k_step<MODE>(kt, rot, KT) * S::BK;
 #pragma unroll
     for (int q = 0; q < S::Q_HI; ++q) {
       const int t = wave + S::NW * q;
