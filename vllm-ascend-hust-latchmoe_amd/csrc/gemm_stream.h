@@ -134,8 +134,13 @@ __device__ __forceinline__ void stream_tile(const StreamArgs& g, char* smem, con
 
   u32x4_t wb[D][RT][2], xb[D][XL];
   // stages past the last load it again (a cached line) and are not multiplied.
-  // Tiles past 64 rows are most often one of several of their slot, whose
-  // weights the next one reads again: these are left in the L2.
+  // Tiles past 64 rows are often one of several of their slot, whose weights
+  // the others read too: these loads are plain ones, which the caches keep.
+  // An expert layer's time, plain against non-temporal (us): H 7168, I 2048,
+  // 257 slots, 2048 tokens with the Zipf(1.1) rank bias (391 row tiles) 4796 /
+  // 5442 (L2 hits 18% against 10% in gate-up, 41 against 29 in down); H 2048, I
+  // 768, 128 slots, 1200 tokens with it 317 / 359, without (one tile of 75 rows
+  // per slot) 268 / 253.
   auto load = [&](int d, int kt) {
     int kr = min(kt, KT - 1) + rot;
     if (kr >= KT) kr -= KT;
@@ -301,20 +306,8 @@ __global__ __launch_bounds__(kStreamWaves * 64, RT == 4 || (RT == 2 && SPLIT) ? 
   }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int slot = __builtin_amdgcn_readfirstlane(stream_tile_slot(g.tile_off, g.P, tile));
-  // the row tile of its slot and the column block
-  int rt = tile - g.tile_off[slot], cb = blockIdx.x;
-  const int nrt = g.tile_off[slot + 1] - g.tile_off[slot];
-  if (nrt > 1 && gridDim.x % 8 == 0) {
-    // a slot of several row tiles: consecutive blocks of an XCD (every eighth
-    // block) take the same weight rows, so that the later tiles find them in
-    // its L2 (kept there: see load).  DeepSeek-V3 expert shape, 2048 tokens
-    // with the Zipf(1.1) rank bias, a layer's experts (us): 5616 -> 5267 with
-    // this order, 4588 with the loads kept as well (320-row tiles: 4749);
-    // without the bias 4356 -> 4328.
-    const int b = rt * gridDim.x + cb;
-    rt = (b >> 3) % nrt;
-    cb = (b >> 3) / nrt * 8 + (b & 7);
-  }
+  const int rt = tile - g.tile_off[slot];  // the row tile of its slot
+  const int cb = blockIdx.x;
   const int p0 = g.offsets[slot] + rt * kStreamBM;
   int n = min(kStreamBM, g.offsets[slot + 1] - p0);
   if (TWO && second) n = min(n, n_pairs - base - p0);
