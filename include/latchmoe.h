@@ -419,6 +419,9 @@ int lmoe_down_combine(const void* act, int T, int H, int I, int k,
  *   streams the slots' rows without a gap;
  *   for more than 16 pairs with a y workspace, else, the down GEMV per (row
  *   block, slot) into y and the combine (three launches).
+ * The GEMVs at every token count, so a token's bits do not depend on its batch;
+ * lmoe_grouped_mlp's LMOE_PATH_STREAM and LMOE_PATH_MFMA add the same products
+ * in other orders, and are the faster ones past a few tokens per slot.
  * With more than 16 pairs y, where given, holds the [T*k, H] bf16 down rows in
  * flat pair order on return.  Each slot's weights are read once however many
  * tokens chose it.  distinct_slots != 0 promises that no slot serves two pairs of one
