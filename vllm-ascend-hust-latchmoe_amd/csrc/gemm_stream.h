@@ -33,12 +33,12 @@
 // leaves twice as many act values off what f64 sums round to (K 2048: 3.4e-4
 // of them, GEMV and SPLIT 1.7e-4; K 7168: 5.7e-4, 2.1e-4, 1.7e-4).
 //
-// Measured (Qwen3 shapes, 128 slots, gate-up + down): 64 tokens 182 us
-// (6.5 TB/s; GEMV 212, 320-row tiles 244), 300 tokens 207 us (247), 1024
-// tokens 245 us (269); DeepSeek-V3 expert shape, 700 tokens 3.56 ms (4.01),
-// 2048 tokens (72 per slot) 4.26 ms (4.59): there the token rows' loads and the
-// output rows' stores take the time past the weight stream's 3.4 ms, not the
-// MFMAs or LDS (a copy without most of the MFMAs: 1% less).
+// Measured, gate-up + down (us): Qwen3 shape, 128 slots, 64 tokens 179 (the
+// 1.18 GB of 125 slots' weights at 6.6 TB/s), 300 tokens 194, 1024 tokens 216 to
+// 231; DeepSeek-V3 expert shape, 257 slots, 700 tokens 3480, 2048 tokens (72 per
+// slot) 4120.  There the token rows' loads and the output rows' stores take the
+// time past the weight stream's 3.3 ms, not the MFMAs or LDS (a copy without
+// most of the MFMAs: 1% less).
 #pragma once
 
 #include "gemm_mfma.h"
@@ -161,8 +161,8 @@ __device__ __forceinline__ void stream_tile(const StreamArgs& g, char* smem, con
 #pragma unroll
   for (int s = 0; s < 2; ++s) roff[s] = r16 * 128 + (((4 * s + kg) ^ stream_swz(r16)) * 16);
   // A wave writes the token tile of stage s only after the barrier of stage
-  // s - 1, which every wave reaches after its
-  // reads of stage s - 2, the last ones of the same buffer.
+  // s - 1, which every wave reaches after its reads of stage s - 2, the last
+  // ones of the same buffer.
   auto multiply = [&](int d, int kt) {
     char* xl = xlds + (kt & 1) * (NG * 2048);
 #pragma unroll
@@ -276,14 +276,18 @@ __device__ __forceinline__ int stream_tile_slot(const int32_t* tile_off, int P, 
   return slot;
 }
 
+// Waves per SIMD that the registers leave: RT 1 four, RT 2 three, with the
+// partial sums three and two (two or three waves take the same time), RT 4 two.
+constexpr int stream_waves(int rt, bool split) {
+  return rt == 4 || (rt == 2 && split) ? 2 : rt == 1 && !split ? 4 : 3;
+}
+
 // grid (blocks of output columns, most row tiles there can be).  TWO: both
 // passes of a decode layer past its bank in one launch, the tiles of g first,
 // then those of g2, whose act rows follow the pairs g places (an overflow
-// slot's rows stay inside the n_pairs rows of the act buffer).  Registers:
-// RT 1 leaves 4 waves per SIMD, RT 2 three, with the partial sums three and two
-// (two or three waves take the same time), RT 4 two.
+// slot's rows stay inside the n_pairs rows of the act buffer).
 template <int MODE, int RT, bool SPLIT, bool TWO>
-__global__ __launch_bounds__(kStreamWaves * 64, RT == 4 || (RT == 2 && SPLIT) ? 2 : RT == 1 && !SPLIT ? 4 : 3) void stream_gemm_kernel(
+__global__ __launch_bounds__(kStreamWaves * 64, stream_waves(RT, SPLIT)) void stream_gemm_kernel(
     StreamArgs g, StreamArgs g2, int n_pairs) {
   __shared__ __attribute__((aligned(1024))) char
       smem[kStreamWaves * RT * 2048 + 2 * (kStreamBM / 16) * 2048];

@@ -5,10 +5,10 @@
 // wave's rows in flight at once; token rows and act rows come from L2.  The
 // down projection is fused with the weighted combine (one workgroup owns R
 // output columns for every token) where the slots serve a pair each or H gives
-// a workgroup to every CU, so the decode layer body is permute + two kernels.  (A single launch would need a cross-block hand-off of act; the
-// agent-scope fences that takes write back / invalidate a whole XCD L2 each
-// and cost far more than a kernel boundary, which in a captured graph is
-// back to back.)
+// a workgroup to every CU, so the decode layer body is permute + two kernels.
+// (A single launch would need a cross-block hand-off of act; the agent-scope
+// fences that takes write back / invalidate a whole XCD L2 each and cost far
+// more than a kernel boundary, which in a captured graph is back to back.)
 // Prefill (hundreds of pairs per slot): bf16 MFMA grouped GEMM, gemm_mfma.h.
 //
 // Reference behaviour: npu_grouped_matmul (GMM1) + npu_swiglu + GMM2 inside
@@ -434,16 +434,16 @@ __global__ __launch_bounds__(256) void down_combine_gemv_kernel(
 
 // ---------------------------------------------------------------------------
 // down GEMV + weighted combine for a few tokens (n_pairs <= kFewPairs), every
-// slot's pairs in one launch: no second kernel that reads y back.  grid ceil(H / (2 RH)):
-// a block owns 2 RH output columns for every active slot, its waves take the
-// slots in list order (heavy slots first) as they become free.  Half wave h
+// slot's pairs in one launch: no second kernel that reads y back.  grid
+// ceil(H / (2 RH)): a block owns 2 RH output columns for every active slot, its
+// waves take the slots in list order (heavy slots first) as they become free.  Half wave h
 // holds rows RH h .. RH h + RH - 1 of the slot's W2 block (DNC 16-byte chunks
 // per lane and row, non-temporal; one contiguous piece of 2 RH rows per slot).
 // Order of a wave's loads: the slot's first act rows, then the next slot's W2
 // rows, so that waiting for the former leaves the latter in flight.  y (bf16
 // values) stays in LDS; the block combines its columns of every token in pair
-// order and, where the caller gave a y, stores it there too.  Every value is formed as in down_rows_kernel and combine_kernel: the
-// same bits.
+// order and, where the caller gave a y, stores it there too.  Every value is
+// formed as in down_rows_kernel and combine_kernel: the same bits.
 // ---------------------------------------------------------------------------
 constexpr int kFewPairs = 256;
 constexpr int kFewWaves = 8;
@@ -911,9 +911,11 @@ static bool part_offsets_fit(const GemmArgs& g, int n_pairs) {
 }
 
 // The wide form (two weight tiles per wave) once its blocks fill the CUs about
-// twice over at three per CU (1500 blocks on 256), else the narrow one, whose twice as many blocks
-// even out the last round: 128 slots of the Qwen3 shape 182 us wide against
-// 190 narrow, 64 slots at 40 tokens 123 against 113 (gate-up + down).
+// twice over at three per CU (1500 blocks on 256), else the narrow one, whose
+// twice as many blocks even out the last round.  Gate-up + down, us, wide /
+// narrow: 128 slots of the Qwen3 shape 64 tokens 185 / 185, 300 tokens 199 /
+// 207; 64 slots, 40 tokens 94 / 95, with skewed routing 80 / 76, 64 tokens 92 /
+// 94, 300 tokens 108 / 121.
 constexpr long long kStreamWideBlocks = 1500;  // per 256 CUs
 constexpr int kStreamWiderRows = 40;
 
@@ -930,11 +932,12 @@ static int launch_stream(const StreamArgs& a, const StreamArgs& b, int n_pairs, 
   if constexpr (MODE == kGateUp && !SPLIT && !TWO) {
     // many rows per slot: twice the weight rows per block, so that a stage
     // loads half the token rows per weight byte, while that still makes two
-    // blocks per CU.  Gate-up, before -> after (us): 257 slots of 72 rows, H
-    // 7168, I 2048: 2788 -> 2665; 64 of 62, H 4096, I 1024: 279 -> 246; 60 of
-    // 47, H 2048, I 1408: 165 -> 156; 128 of 64, H 2048, I 768: the same.  With
-    // fewer rows it is slower (128 of 19: 145 -> 157; 257 of 10: 2294 -> 2345),
-    // and the down GEMM (more output rows to store) gains nothing.
+    // blocks per CU.  Gate-up, without -> with it (us): 257 slots of 72 rows, H
+    // 7168, I 2048: 2708 -> 2594; 64 of 62, H 4096, I 1024: 232 -> 190; 60 of
+    // 47, H 2048, I 1408: 132 -> 120; 128 of 62, H 2048, I 768: 147 -> 139 (with
+    // skewed routing 173 -> 177).  With fewer rows it is slower (128 of 19: 122
+    // -> 125; 257 of 10: 2179 -> 2219; 64 of 19, H 4096: 174 -> 183), and the
+    // down GEMM (more output rows to store) gains nothing.
     const int wider = (a.N + 2 * wide_cols - 1) / (2 * wide_cols);
     if (pass_pairs >= kStreamWiderRows * static_cast<long long>(a.P) &&
         static_cast<long long>(wider) * max_active >= 2 * device_cus()) {

@@ -222,11 +222,11 @@ def _overflow_pass(hidden, topk_ids, k: int, overflow: PreparedSlotWeights, ws: 
 def _merged_passes(hidden, k: int, w13_slots, overflow: PreparedSlotWeights, path: int) -> bool:
     """Whether an overflow layer runs both passes in shared launches: the
     decode GEMV path with rows of at most TWO_PASS_MAX_COLS columns
-    (decode_mlp_two_passes), or the weight-streaming kernel in both (stream_mlp_two_passes).  In the
-    48-layer B=64 decode graph (Qwen3-30B-A3B shapes, ~33 of 48 layers with
-    an overflow pass) shared GEMV launches took the layer from 186.0 to
-    180.2 us, and both tables' builds in one permutation launch on top of
-    them to 176.0 us (same box)."""
+    (decode_mlp_two_passes), or the weight-streaming kernel in both
+    (stream_mlp_two_passes).  When the 48-layer B=64 decode graph (Qwen3-30B-A3B
+    shapes, ~33 of 48 layers with an overflow pass) ran the GEMVs, shared
+    launches took the layer from 186.0 to 180.2 us, and both tables' builds in
+    one permutation launch on top of them to 176.0 us (same box)."""
     if path == native.LMOE_PATH_GEMV:
         return hidden.shape[1] <= native.TWO_PASS_MAX_COLS and \
             int(w13_slots.shape[1]) // 2 <= native.TWO_PASS_MAX_COLS

@@ -646,16 +646,21 @@ GEMV_MAX_PAIRS_PER_EXPERT_WHOLE = 2.75
 GEMV_WHOLE_HIDDEN = (1024, 2048, 4096)
 GEMV_WHOLE_INTERMEDIATE = (512, 768, 1024, 2048, 4096)
 # Most pairs per slot, on average, of a pass on STREAM_BLOCK_M-row tiles: past
-# one tile per slot the second one costs as much as the wider tiles do.
-# Streaming against the 320-row tiles (us): Qwen3 shape 1024 tokens (64 pairs
-# per slot) 245 / 269, 1300 (81) 272 / 274, 1600 (100) 400 / 285, with half the
-# rank bias 800 tokens 269 / 317, 1300 330 / 341; Qwen1.5-MoE, the same bias,
-# 400 tokens (27 pairs) 210 / 246, 800 (53) 267 / 258; DeepSeek-V3 shape 1024
-# tokens (36 pairs) 3734 / 4127, 2048 (72) 4341 / 4590.  With the whole rank
-# bias, hot slots of several tiles sharing their weights through the L2: Qwen3
-# 600 tokens 247 / 289, 1200 318 / 363; Qwen1.5-MoE 800 258 / 286, 1100 (73
-# pairs) 294 / 299; DeepSeek-V3 1100 3851 / 4116, 2048 4579 / 4749.  Equal
-# near the line without a bias (Qwen1.5-MoE, 1100 tokens 243 / 240).
+# one tile per slot the second one costs as much as the wider tiles do.  A
+# layer's experts, streaming / 320-row tiles, us (tokens, pairs per slot):
+#   Qwen3 shape   no rank bias  300 (19) 211 / 242, 1024 (64) 254 / 271, 1200 (75) 270 / 278, 1300 (81) 302 / 281
+#                 half of it    300 228 / 260, 800 (50) 262 / 321, 1200 307 / 348, 1300 329 / 351
+#                 Zipf(1.1)     300 216 / 287, 600 (38) 245 / 287, 1200 316 / 362
+#   Qwen1.5-MoE   no rank bias  300 (20) 195 / 217, 800 (53) 212 / 234, 1100 (73) 244 / 243
+#                 half of it    400 (27) 207 / 257, 800 252 / 269, 1100 281 / 288
+#                 Zipf(1.1)     800 259 / 284, 1100 294 / 301
+#   DeepSeek-V3   no rank bias  700 (25) 3522 / 3997, 1024 (36) 3803 / 4241, 2048 (72) 4331 / 4761
+#                 half of it    1100 (39) 4048 / 4399, 2048 4772 / 4737
+#                 Zipf(1.1)     1100 4018 / 4262, 2048 4867 / 5033
+# The average is all that the host knows.  Where the routing leaves most slots
+# without a pair the others hold more than it says and the wide tiles would be
+# faster: 1100 tokens of the Qwen3 shape on 32 of its 128 experts (275 pairs
+# each) 199 / 138, on 64 of them 252 / 205; 600 tokens on 32 125 / 112.
 STREAM_MAX_PAIRS_PER_SLOT = 75
 
 
@@ -1111,9 +1116,11 @@ def fused_moe_decode(
     """Decode layer body: gate_up GEMV, then down GEMV fused with the combine
     (up to 16 pairs, no y, or up to 256 pairs where H gives about one workgroup
     per CU), or with a [T*k, H] bf16 workspace y and more pairs the down GEMV
-    per (row block, slot) into y and the combine; same out either way.  distinct_slots: the caller promises that no slot serves two
-    pairs of one token (router-fed ids through a slot table); with one token
-    it selects the faster one-pair-per-slot kernels."""
+    per (row block, slot) into y and the combine; same out either way.  The
+    GEMVs at every token count (fused_moe.fused_experts leaves them where
+    layer_path does).  distinct_slots: the caller promises that no slot serves
+    two pairs of one token (router-fed ids through a slot table); with one
+    token it selects the faster one-pair-per-slot kernels."""
     lib = load_library()
     _need(x, "x", torch.bfloat16)
     T, H = x.shape
